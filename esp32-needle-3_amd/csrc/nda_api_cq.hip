@@ -169,8 +169,10 @@ int nda_cq_gemm(const nda_cq *t, uint32_t rows, const float *xh, float *y, void 
 static bool cq_split_ok(const nda_cq *t) { return t->bits == 2 && t->group >= 32; }
 static bool cq_lut2_ok(const nda_cq *t) { return t->bits == 2 && t->in_pad <= (uint32_t)CQ_LUT_MAX_IN; }
 
-int nda_cq_gemv_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const float *xh, float *const *ys,
-                     void *stream)
+// raw: xh holds the raw activations [rows][in], which the kernel prepares
+// itself (group 128); the bits of y are the same.
+static int cq_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const float *xh, bool raw,
+                   float *const *ys, void *stream)
 {
     if (!ts || !ys || n == 0 || n > (uint32_t)CQ_MAX_T || (rows && !xh) || ((uintptr_t)xh & 15))
         return NDA_ERR_ARG;
@@ -183,6 +185,8 @@ int nda_cq_gemv_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const f
     a.xh = xh;
     a.rows = rows;
     a.in_pad = t0->in_pad;
+    a.in = t0->in;
+    a.scale = 1.0f / sqrtf((float)t0->group);
     a.group = t0->group;
     a.ngroup = t0->ngroup;
     a.bits = t0->bits;
@@ -206,7 +210,13 @@ int nda_cq_gemv_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const f
         tiles += (t->out + CQ_LUT_OT - 1) / CQ_LUT_OT;
     }
     a.tile0[n] = tiles;
-    return launch_cq_lut2(a, (hipStream_t)stream) == hipSuccess ? NDA_OK : NDA_ERR_HIP;
+    return launch_cq_lut2(a, raw, (hipStream_t)stream) == hipSuccess ? NDA_OK : NDA_ERR_HIP;
+}
+
+int nda_cq_gemv_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const float *xh, float *const *ys,
+                     void *stream)
+{
+    return cq_lut2(ts, n, rows, xh, false, ys, stream);
 }
 
 // rows rounded up to a block of 32: operand blocks (4 bytes per element), then the exponents
@@ -297,10 +307,13 @@ static int cq_project(const nda_cq *const *ts, uint32_t n, uint32_t rows, const 
         split = split && cq_split_ok(ts[i]);
         lut = lut && cq_lut2_ok(ts[i]);
     }
+    // group 128 (the archive's): one launch, the rows prepared inside it
+    if (lut && ts[0]->group == 128)
+        return cq_lut2(ts, n, rows, x, true, ys, st);
     if (lut) {
         if (int rc = nda_cq_prepare(ts[0], rows, x, (float *)xs, st))
             return rc;
-        return nda_cq_gemv_lut2(ts, n, rows, (const float *)xs, ys, st);
+        return cq_lut2(ts, n, rows, (const float *)xs, false, ys, st);
     }
     if (split) {
         if (int rc = nda_cq_prepare_split(ts[0], rows, x, xs, st))

@@ -801,64 +801,159 @@ void cq_gemm_split_kernel(CqSplitArgs a)
 // row the pair table T[p][i0 + 4 i1] = cb[i0] xh[2p] + cb[i1] xh[2p+1] in
 // LDS; per output the groups in order, each group's 32-bit words in order,
 // nibble k of a word added into accumulator k % 4 from table block k, and
-// acc = acc + norm * ((s0 + s1) + (s2 + s3)). One work-group per
-// (256-output tile, row), one output per thread; every product and sum
-// rounds on its own.
-__global__ __launch_bounds__(256) void cq_lut2_kernel(CqGemmArgs a)
+// acc = acc + norm * ((s0 + s1) + (s2 + s3)); every product and sum rounds
+// on its own.
+//
+// What bounds it is the serial chain of one output, not bytes (the codes of
+// all outputs are 0.3 MB): 384 lookups and 96 dependent additions at 768
+// inputs. Only the last line of the recipe ties the groups together, so a
+// work-group is 64 outputs (one per lane) of one row with one wave per
+// group: each wave builds its own group's table (no barrier), walks its
+// group's words and leaves norm * sum in LDS, and the first wave adds the
+// groups up in order. The chain is a sixth as long, and 1568 outputs are 25
+// work-groups a row instead of 8.
+// G: the group at compile time, 0: at run time. PREP (group 128): xh holds
+// the raw activations and each wave transforms its own group in registers,
+// lane l columns 2l and 2l + 1, the engine's butterflies stage by stage as in
+// cq_prepare_split_reg_kernel; a launch less, and 7 stages of one value pair
+// a lane cost less than the row's round trip through memory.
+// Per launch at 768 inputs, group 128 (q/k/v/gate, 1568 outputs): 4.9 us for
+// 1 row and 7.0 us for 24, where a work-group of 256 outputs with a whole
+// chain per thread took 21.1 and 21.6 us, after a prepare launch of 4.1-4.8.
+template <int G, bool PREP>
+__global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmArgs a)
 {
 #pragma clang fp contract(off)
-    extern __shared__ float lut[];   // [in_pad / 2][16]
+    extern __shared__ __attribute__((aligned(16))) float lut[];   // [waves][group / 2][16], then [ngroup][64]
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const uint32_t group = G ? G : a.group, gw = group / 16;      // words per group
     const uint32_t tile = blockIdx.x, row = blockIdx.y;
     uint32_t t = 0;
     while (t + 1 < a.nt && tile >= a.tile0[t + 1])
         t++;
-    const float *xh = a.xh + (uint64_t)row * a.in_pad;
-    const float *cb = a.cb[t];
-    for (uint32_t e = threadIdx.x; e < a.in_pad * 8; e += 256) {
-        const uint32_t p = e >> 4;
-        const float x0 = xh[2 * p], x1 = xh[2 * p + 1];
-        const float lo = cb[e & 3] * x0, hi = cb[(e >> 2) & 3] * x1;
-        lut[e] = lo + hi;
-    }
-    __syncthreads();
-    const uint32_t o = (tile - a.tile0[t]) * CQ_LUT_OT + threadIdx.x;
-    if (o >= a.out[t])
-        return;
-    const uint32_t *q = reinterpret_cast<const uint32_t *>(a.packed[t] + (uint64_t)o * a.rowbytes);
-    const uint16_t *nrm = a.norms[t] + (uint64_t)o * a.ngroup;
-    const uint32_t gw = a.group / 16;          // words per group
-    const float *T = lut;
+    const uint32_t o = (tile - a.tile0[t]) * CQ_LUT_OT + lane, oc = min(o, a.out[t] - 1);
+    const uint32_t *qw = reinterpret_cast<const uint32_t *>(a.packed[t] + (uint64_t)oc * a.rowbytes);
+    const uint16_t *nrm = a.norms[t] + (uint64_t)oc * a.ngroup;
+    const float cb[4] = {a.cb[t][0], a.cb[t][1], a.cb[t][2], a.cb[t][3]};
+    float *const T0 = lut + wave * group * 8;
+    float *const part = lut + nw * group * 8;
     float acc = 0.0f;
-    for (uint32_t gi = 0; gi < a.ngroup; gi++) {
+    for (uint32_t gi = wave; gi < a.ngroup; gi += nw) {
         const float nf = half_bits_to_float(nrm[gi]);
-        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-        for (uint32_t j = 0; j < gw; j++) {
-            const uint32_t w = q[j];
-            s0 = s0 + T[w & 15u];
-            s1 = s1 + T[16 + ((w >> 4) & 15u)];
-            s2 = s2 + T[32 + ((w >> 8) & 15u)];
-            s3 = s3 + T[48 + ((w >> 12) & 15u)];
-            T += 64;
-            s0 = s0 + T[(w >> 16) & 15u];
-            s1 = s1 + T[16 + ((w >> 20) & 15u)];
-            s2 = s2 + T[32 + ((w >> 24) & 15u)];
-            s3 = s3 + T[48 + (w >> 28)];
-            T += 64;
-        }
-        q += gw;
-        acc = acc + nf * ((s0 + s1) + (s2 + s3));
+        const uint32_t *q = qw + gi * gw;
+        uint32_t w[G ? G / 16 : 1];
+        if constexpr (G != 0)
+#pragma unroll
+            for (int j = 0; j < G / 64; j++) {         // rows and groups are 16-byte multiples
+                const uint4 v = reinterpret_cast<const uint4 *>(q)[j];
+                w[4 * j] = v.x;
+                w[4 * j + 1] = v.y;
+                w[4 * j + 2] = v.z;
+                w[4 * j + 3] = v.w;
+            }
+        for (uint32_t p = lane; p < group / 2; p += 64) {
+            float x0, x1;
+            if constexpr (PREP) {
+                const uint32_t c = gi * G + 2 * p;
+                const float *x = a.xh + (uint64_t)row * a.in;
+                const float u = c < a.in ? x[c] : 0.0f, v = c + 1 < a.in ? x[c + 1] : 0.0f;
+                x0 = u + v;
+                x1 = u - v;
+                // lengths 2 .. 64: lanes l and l ^ (len / 2); lower lane
+                // v + w, upper w - v (one rounding either way)
+#define NDA_STAGE(M)                                                     \
+    {                                                                    \
+        const float sg = (lane & M) ? -1.0f : 1.0f;                      \
+        const float w0 = xor_lanes<M>(x0, lane), w1 = xor_lanes<M>(x1, lane); \
+        x0 = fmaf(sg, x0, w0);                                           \
+        x1 = fmaf(sg, x1, w1);                                           \
     }
-    a.y[t][(uint64_t)row * a.out[t] + o] = acc;
+                NDA_STAGE(1)
+                NDA_STAGE(2)
+                NDA_STAGE(4)
+                NDA_STAGE(8)
+                NDA_STAGE(16)
+                NDA_STAGE(32)
+#undef NDA_STAGE
+                x0 = x0 * a.scale;
+                x1 = x1 * a.scale;
+            } else {
+                const float2 v = *reinterpret_cast<const float2 *>(a.xh + (uint64_t)row * a.in_pad + gi * group + 2 * p);
+                x0 = v.x;
+                x1 = v.y;
+            }
+            float l[4], h[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                l[i] = cb[i] * x0;
+                h[i] = cb[i] * x1;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                *reinterpret_cast<float4 *>(T0 + 16 * p + 4 * i) =
+                    float4{l[0] + h[i], l[1] + h[i], l[2] + h[i], l[3] + h[i]};
+        }
+        // a wave's LDS operations complete in order: its own table needs no barrier
+        __builtin_amdgcn_wave_barrier();
+        const float *T = T0;
+        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+        auto word = [&](uint32_t v) __attribute__((always_inline)) {
+            s0 = s0 + T[v & 15u];
+            s1 = s1 + T[16 + ((v >> 4) & 15u)];
+            s2 = s2 + T[32 + ((v >> 8) & 15u)];
+            s3 = s3 + T[48 + ((v >> 12) & 15u)];
+            s0 = s0 + T[64 + ((v >> 16) & 15u)];
+            s1 = s1 + T[80 + ((v >> 20) & 15u)];
+            s2 = s2 + T[96 + ((v >> 24) & 15u)];
+            s3 = s3 + T[112 + (v >> 28)];
+            T += 128;
+        };
+        if constexpr (G != 0) {
+#pragma unroll
+            for (int j = 0; j < G / 16; j++)
+                word(w[j]);
+        } else {
+            for (uint32_t j = 0; j < gw; j++)
+                word(q[j]);
+        }
+        const float r = nf * ((s0 + s1) + (s2 + s3));
+        if (nw > 1)
+            part[gi * 64 + lane] = r;
+        else
+            acc = acc + r;
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (nw > 1) {
+        __syncthreads();
+        if (wave)
+            return;
+        for (uint32_t gi = 0; gi < a.ngroup; gi++)
+            acc = acc + part[gi * 64 + lane];
+    }
+    if (o < a.out[t])
+        a.y[t][(uint64_t)row * a.out[t] + o] = acc;
 }
 
-hipError_t launch_cq_lut2(const CqGemmArgs &a, hipStream_t s)
+hipError_t launch_cq_lut2(const CqGemmArgs &a, bool prep, hipStream_t s)
 {
     if (a.rows == 0 || a.nt == 0 || a.tile0[a.nt] == 0)
         return hipSuccess;
-    if (a.bits != 2 || a.group % 16 || a.in_pad > CQ_LUT_MAX_IN || a.rows > 65535)
+    if (a.bits != 2 || a.group % 16 || a.in_pad > CQ_LUT_MAX_IN || a.rows > 65535 || (prep && a.group != 128))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(cq_lut2_kernel, dim3(a.tile0[a.nt], a.rows), dim3(256), (size_t)a.in_pad * 8 * sizeof(float),
-                       s, a);
+    // one wave per group as far as 64 KiB of LDS hold their tables (and,
+    // with several waves, the groups' sums); a single wave keeps its sum in
+    // a register
+    const uint32_t tab = a.group * 8 * sizeof(float), sums = a.ngroup * 64 * sizeof(float);
+    const uint32_t nw = std::max(1u, std::min({a.ngroup, (uint32_t)CQ_LUT_MAX_WAVES, (65536u - sums) / tab}));
+    const size_t lds = (size_t)nw * tab + (nw > 1 ? sums : 0);
+    const dim3 grid(a.tile0[a.nt], a.rows), wg(64 * nw);
+    if (prep)
+        hipLaunchKernelGGL((cq_lut2_kernel<128, true>), grid, wg, lds, s, a);
+    else if (a.group == 128)
+        hipLaunchKernelGGL((cq_lut2_kernel<128, false>), grid, wg, lds, s, a);
+    else
+        hipLaunchKernelGGL((cq_lut2_kernel<0, false>), grid, wg, lds, s, a);
     return hipGetLastError();
 }
 

@@ -182,10 +182,12 @@ struct CqPrepArgs {
  * bits) in one launch: the grid walks their output tiles in order (64
  * outputs per tile in the GEMM, CQ_LUT_OT in the engine-order kernel). */
 constexpr int CQ_MAX_T = 8;
-constexpr int CQ_LUT_OT = 256;        /* engine-order kernel: outputs per work-group */
+constexpr int CQ_LUT_OT = 64;         /* engine-order kernel: outputs per work-group */
+constexpr int CQ_LUT_MAX_WAVES = 16;  /*   and its waves at most, each on groups of its own */
 constexpr int CQ_LUT_MAX_IN = 2048;   /* its pair table, in_pad * 32 bytes of LDS, within 64 KiB */
 struct CqGemmArgs {
-    const float *xh;                    /* [rows][in_pad] prepared activations */
+    const float *xh;                    /* [rows][in_pad] prepared activations (engine-order kernel from
+                                           raw ones: [rows][in]) */
     float *y[CQ_MAX_T];                 /* [rows][out[t]] */
     const uint8_t *packed[CQ_MAX_T];    /* [out][rowbytes] LSB-first index bitstream */
     const uint16_t *norms[CQ_MAX_T];    /* [out][ngroup] fp16 bits */
@@ -194,6 +196,8 @@ struct CqGemmArgs {
     uint32_t tile0[CQ_MAX_T + 1];       /* first grid.y tile of each tensor; tile0[nt] = total */
     uint32_t nt;
     uint32_t rows, in_pad, group, ngroup, bits, rowbytes;
+    uint32_t in;                        /* raw activations: their width, and 1 / sqrt(group) */
+    float scale;
 };
 
 /* The split-precision form of a prepared activation: xh * 2^rexp[r] as an
@@ -243,7 +247,8 @@ constexpr int CQ_SPLIT_NT = 64 * CQ_SPLIT_OB;   /* outputs per work-group */
 
 hipError_t launch_cq_prepare(const CqPrepArgs &a, hipStream_t s);
 hipError_t launch_cq_gemm(const CqGemmArgs &a, hipStream_t s);
-hipError_t launch_cq_lut2(const CqGemmArgs &a, hipStream_t s);
+/* prep: a.xh holds the raw activations (group 128 only) */
+hipError_t launch_cq_lut2(const CqGemmArgs &a, bool prep, hipStream_t s);
 hipError_t launch_cq_prepare_split(const CqPrepSplitArgs &a, hipStream_t s);
 hipError_t launch_cq_gemm_split(const CqSplitArgs &a, hipStream_t s);
 hipError_t launch_cq_split_tables(const CqTabArgs &a, hipStream_t s);

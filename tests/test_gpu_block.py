@@ -155,3 +155,44 @@ def test_block_batched(shape, kv_dtype):
     for layer in cqs:
         for c in layer:
             c.close()
+
+
+@pytest.mark.parametrize("dm,group,rows", [(768, 128, 64), (333, 128, 1), (130, 128, 7), (2047, 128, 3), (256, 64, 5)])
+def test_block_projections_equal_the_separate_calls(dm, group, rows):
+    """The block's projections of a few rows (at group 128 one launch from
+    the raw activations, odd and padded widths included) equal
+    nda_cq_prepare + nda_cq_gemv_lut2 bit for bit: the same attention over
+    them, so the block's output does too."""
+    N = nda()
+    say("block projections", dm, group, rows)
+    nh, nkv, qk, vd = 12, 2, 48, 64
+    rng = np.random.default_rng(dm + rows)
+    cb = (np.sort(rng.standard_normal(4)) / np.sqrt(group)).astype(np.float32)
+
+    def tensor(o, i):
+        pad = (i + group - 1) // group * group
+        packed = rng.integers(0, 256, o * pad // 4, dtype=np.uint8)
+        norms = rng.uniform(0.25, 2.0, (o, pad // group)).astype(np.float16)
+        return N.CQ(o, i, group, 2, np.concatenate([packed, norms.view(np.uint8).ravel()]), cb)
+
+    outs = [nh * qk, nkv * qk, nkv * vd, nh * vd]
+    ts = [tensor(o, dm) for o in outs] + [tensor(dm, nh * vd)]
+    ctx = N.Context(1, nh, nkv, qk, vd, 64, kv_dtype=O.KV_INT8, max_seqs=rows)
+    ctx.block_weights(0, *ts)
+    x = N.DevBuf.from_array(rng.standard_normal((rows, dm)).astype(np.float32))
+    got, want = N.DevBuf(rows * dm * 4), N.DevBuf(rows * dm * 4)
+    ctx.attention_block(0, rows, x, got)
+    xh, ah = N.DevBuf(rows * ts[0].in_pad * 4), N.DevBuf(rows * ts[4].in_pad * 4)
+    q, k, v, g = (N.DevBuf(rows * o * 4) for o in outs)
+    att = N.DevBuf(rows * nh * vd * 4)
+    ts[0].prepare(rows, x, xh)
+    N.cq_gemv_lut2(ts[:4], rows, xh, [q, k, v, g])
+    ctx.step(0, rows, q, k, v, att, gate=g)
+    ts[4].prepare(rows, att, ah)
+    N.cq_gemv_lut2(ts[4:], rows, ah, [want])
+    N.device_sync()
+    a, b = (t.to_array(np.uint32, (rows, dm)) for t in (got, want))
+    assert np.array_equal(a, b), int((a != b).sum())
+    ctx.close()
+    for t in ts:
+        t.close()
