@@ -606,7 +606,7 @@ void nda_destroy(nda_ctx *c)
     if (c->h_ring)
         (void)hipHostFree(c->h_ring);
     void *bufs[] = {c->pool, c->d_pages, c->d_prefix_pages, c->d_seqs, c->d_rows, c->d_part,
-                    c->d_stage, c->d_pf, c->d_hist, c->d_snap_hist, c->d_prefix_hist,
+                    c->d_stage, c->d_pf, c->d_pf_part, c->d_hist, c->d_snap_hist, c->d_prefix_hist,
                     c->d_front_w, c->d_front_norm, c->d_rope, c->d_qfront, c->d_front_rows,
                     c->d_hist_ops, c->d_bscr, c->d_order};
     for (void *b : bufs)

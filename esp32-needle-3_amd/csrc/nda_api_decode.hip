@@ -307,6 +307,7 @@ static int prefix_pass(nda_ctx *c, const AttnArgs &a, uint32_t nseq, const uint3
     pa.items = c->d_pf;
     pa.part = a.part;
     pa.max_chunks = a.max_chunks;
+    pa.part_stride = c->cfg.v_head_dim + 2;
     pa.tab_cap = (ps.n_sh + 31) / 32;         // the prefix's tiles only
     pa.pg = a.pg;
     pa.n_items = (uint32_t)(items.size() / 8);

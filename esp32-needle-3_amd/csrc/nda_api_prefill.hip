@@ -33,26 +33,61 @@ int prefill_check(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t
 // eight ranges; each range is padded to the longest with empty items. A
 // launch of ragged chunks (L ~ U[8K, 32K]) then ends on short items on
 // every XCD, rather than on whichever long items came last. A group's row
-// tiles stay adjacent in one range, where L2 serves their shared K/V.
+// tiles stay adjacent in one range, where L2 serves their shared K/V. Fewer
+// groups than two per range (one GQA prompt) would leave XCDs idle: their row
+// tiles are dealt one by one. A bin holds (batch index, kv-head, row tile).
 static uint32_t prefill_bins(const nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens,
-                             uint32_t rep, uint32_t trows, std::vector<std::pair<uint32_t, uint32_t>> (&bins)[8])
+                             uint32_t rep, uint32_t trows, std::vector<std::array<uint32_t, 3>> (&bins)[8],
+                             size_t *total = nullptr)
 {
     std::vector<std::pair<uint64_t, uint32_t>> key;      // (keys visited, batch index)
     for (uint32_t b = 0; b < nseq; b++)
         if (n_tokens[b])
             key.push_back({(uint64_t)c->seqs[sid(ids, b)].pos + n_tokens[b], b});
     std::stable_sort(key.begin(), key.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
-    uint32_t load[8] = {}, rank = 0;
+    const bool single = key.size() * c->cfg.n_kv_heads < 16;
+    uint32_t rank = 0;
+    size_t n = 0, most = 0;
     for (auto &bin : bins)
         bin.clear();
     for (const auto &kb : key) {
         const uint32_t nt = (n_tokens[kb.second] * rep + trows - 1) / trows;
-        for (uint32_t g = 0; g < c->cfg.n_kv_heads; g++, rank++) {
-            bins[rank % 8].push_back({kb.second, g});
-            load[rank % 8] += nt;
-        }
+        for (uint32_t g = 0; g < c->cfg.n_kv_heads; g++, rank += !single)
+            for (uint32_t t = 0; t < nt; t++, rank += single)
+                bins[rank % 8].push_back({kb.second, g, t});
     }
-    return *std::max_element(load, load + 8);
+    for (const auto &bin : bins) {
+        n += bin.size();
+        most = std::max(most, bin.size());
+    }
+    if (total)
+        *total = n;
+    return (uint32_t)most;
+}
+
+// Parts to split every item's key tiles into, so that a launch of few items
+// (one prompt, a few long documents) fills the chip: each part is a
+// work-group of its own, and a merge launch follows. Measured over 1-64
+// sequences, 16-512 tokens, 0-20K stored positions (us, whole -> split):
+//   - parts up to the waves the chip holds (16 per CU; past about 64 tiles,
+//     where the tiles outweigh the states' traffic, half of that below): 16
+//     heads x 512 tokens over 18K positions 449 -> 44 (16 parts), over 4.5K
+//     128 -> 28; 56 items over 18K 552 -> 137 (8 parts); 248 items 171 -> 149
+//     (2 parts, 4 parts 153);
+//   - at least 2 tiles a part (8 past 16 parts), and 12 tiles in all: the
+//     merge costs 4-5 us, a tile about 1.1 (8 tiles: 13.5 -> 12.2 at best,
+//     and 2-5 tiles 6 -> 11; 12 tiles 18 -> 13);
+//   - below 32 tiles, 4 parts or none: 128 items of 20 tiles took 26.5 whole
+//     and 26.9 in 2 parts.
+static uint32_t prefill_ksplit(const nda_ctx *c, size_t items, uint32_t tiles, int waves)
+{
+    if (items == 0 || tiles < 12)
+        return 0;
+    const size_t slots = (size_t)c->cus * (tiles >= 64 ? 16 : 8) / (items * (size_t)waves);
+    uint32_t parts = 1;
+    while (parts < PF_MAX_PARTS && 2 * parts <= slots && tiles / (2 * parts) >= (parts >= 16 ? 8u : 2u))
+        parts *= 2;
+    return parts >= (tiles < 32 ? 4u : 2u) ? parts : 0;
 }
 
 int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens, PrefillPlan &pl)
@@ -62,6 +97,11 @@ int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t 
     for (uint32_t b = 0; b < nseq; b++) {
         const SeqHost &s = c->seqs[sid(ids, b)];
         if (n_tokens[b]) {
+            // key tiles of the sequence's longest item (its work-group's tile
+            // table): the shared prefix's, then the own slots up to the
+            // chunk's last token
+            const uint32_t n_sh = visible(s, s.pos, c->cfg.window).n_sh;
+            pl.tab_cap = std::max<uint32_t>(pl.tab_cap, (n_sh + 31) / 32 + (s.pos + n_tokens[b] - n_sh + 31) / 32);
             const Vis v = visible(s, s.pos + n_tokens[b] - 1, c->cfg.window);
             pl.max_total = std::max(pl.max_total, v.n_sh + v.n_own);
             pl.sum_total += (uint64_t)n_tokens[b] * (v.n_sh + v.n_own);
@@ -87,14 +127,18 @@ int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t 
     pl.waves = NDA_PF_FORCE_W;
 #endif
     pl.trows = 32u * pl.waves;
-    std::vector<std::pair<uint32_t, uint32_t>> bins[8];
-    pl.n_items = 8 * (size_t)prefill_bins(c, nseq, ids, n_tokens, pl.rep, pl.trows, bins);
+    std::vector<std::array<uint32_t, 3>> bins[8];
+    size_t items = 0;
+    pl.n_items = 8 * (size_t)prefill_bins(c, nseq, ids, n_tokens, pl.rep, pl.trows, bins, &items);
+    if (!pl.valu)
+        pl.ksplit = prefill_ksplit(c, items, pl.tab_cap, pl.waves);
     return NDA_OK;
 }
 
 // The device buffers a planned prefill needs: row staging and either the
-// partials of split VALU rows or the MFMA work list.
-int prefill_reserve(nda_ctx *c, const PrefillPlan &pl)
+// partials of split VALU rows or the MFMA work list. A split-key plan whose
+// parts get no memory runs unsplit.
+int prefill_reserve(nda_ctx *c, PrefillPlan &pl)
 {
     if (pl.rows == 0)
         return NDA_OK;
@@ -102,7 +146,12 @@ int prefill_reserve(nda_ctx *c, const PrefillPlan &pl)
         return reserve_attend(c, (uint32_t)pl.rows, true, pl.max_total, pl.sum_total);
     if (int rc = ensure_rows(c, pl.rows))
         return rc;
-    return ensure_pf(c, 8 * pl.n_items);
+    if (int rc = ensure_pf(c, 8 * pl.n_items))
+        return rc;
+    if (pl.ksplit &&
+        ensure_buf(c, c->d_pf_part, c->pf_part_cap, pl.rows * c->cfg.n_heads * pl.ksplit * PF_PART_STRIDE))
+        pl.ksplit = 0;
+    return NDA_OK;
 }
 
 } // namespace nda_host
@@ -196,27 +245,19 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
         tok0[b] = tok;
         tok += n_tokens[b];
     }
-    std::vector<std::pair<uint32_t, uint32_t>> bins[8];
+    std::vector<std::array<uint32_t, 3>> bins[8];
     const uint32_t per_bin = prefill_bins(c, nseq, ids, n_tokens, rep, trows, bins);
     std::vector<uint32_t> items;
     items.reserve(8 * 8 * (size_t)per_bin);
-    // key tiles of the longest item (its work-group's tile table): the
-    // shared prefix's, then the own slots up to the chunk's last token
-    uint32_t tab_cap = 0;
     for (const auto &bin : bins) {
-        uint32_t n = 0;
-        for (const auto &bg : bin) {
-            const uint32_t b = bg.first, qq = sid(ids, b);
+        for (const auto &it : bin) {
+            const uint32_t b = it[0], qq = sid(ids, b);
             const SeqHost &s = c->seqs[qq];
             const Vis v = visible(s, s.pos, c->cfg.window);
-            tab_cap = std::max<uint32_t>(tab_cap, (v.n_sh + 31) / 32 + (s.pos + n_tokens[b] - v.n_sh + 31) / 32);
-            const uint32_t nt = (n_tokens[b] * rep + trows - 1) / trows;
-            for (uint32_t t = 0; t < nt; t++, n++) {
-                const uint32_t rec[8] = {qq, bg.second, t, tok0[b], n_tokens[b], s.pos, v.n_sh, (uint32_t)s.prefix};
-                items.insert(items.end(), rec, rec + 8);
-            }
+            const uint32_t rec[8] = {qq, it[1], it[2], tok0[b], n_tokens[b], s.pos, v.n_sh, (uint32_t)s.prefix};
+            items.insert(items.end(), rec, rec + 8);
         }
-        for (; n < per_bin; n++) {
+        for (size_t n = bin.size(); n < per_bin; n++) {
             const uint32_t pad[8] = {0xFFFFFFFFu, 0, 0, 0, 0, 0, 0, 0};
             items.insert(items.end(), pad, pad + 8);
         }
@@ -234,7 +275,13 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
     pa.prefix_pages = c->d_prefix_pages;
     pa.seqs = c->d_seqs;
     pa.items = c->d_pf;
-    pa.tab_cap = tab_cap;
+    pa.tab_cap = pl.tab_cap;
+    if (pl.ksplit) {
+        pa.tab_cap = (pl.tab_cap + pl.ksplit - 1) / pl.ksplit;
+        pa.ksplit = pa.max_chunks = pl.ksplit;
+        pa.part = c->d_pf_part;
+        pa.part_stride = PF_PART_STRIDE;
+    }
     pa.pg = c->pg;
     pa.n_items = (uint32_t)(items.size() / 8);
     pa.nh = c->cfg.n_heads;
@@ -243,6 +290,9 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
     hipError_t e = launch_prefill(c->geo, pa, waves, st);
     if (e != hipSuccess)
         return hip_fail(c, e, "prefill kernel launch");
+    if (pl.ksplit)
+        if (hipError_t e2 = launch_pf_merge(pa, rows * c->cfg.n_heads, st); e2 != hipSuccess)
+            return hip_fail(c, e2, "prefill merge launch");
     return NDA_OK;
 }
 

@@ -68,6 +68,8 @@ struct nda_ctx {
     size_t stage_cap = 0;
     uint32_t *d_pf = nullptr;           // prefill work list staging
     size_t pf_cap = 0;                  // uint32 entries
+    float *d_pf_part = nullptr;         // states of a split-key prefill
+    size_t pf_part_cap = 0;             // floats
     // GQA decode work order (longest rows first) for batches of sequences
     // 0..rows-1, valid while no sequence state has changed since it was built
     uint32_t *d_order = nullptr;
@@ -288,10 +290,14 @@ struct PrefillPlan {
     int waves = 4;
     bool valu = false;
     size_t n_items = 0;
+    uint32_t tab_cap = 0;               // key tiles of the longest item
+    uint32_t ksplit = 0;                // parts per item's key tiles (0: whole)
 };
+constexpr uint32_t PF_MAX_PARTS = 64;
+constexpr uint32_t PF_PART_STRIDE = 68; // a split part's floats: 64 sums, max, weight sum, padded to 16 bytes
 int prefill_check(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens);
 int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens, PrefillPlan &pl);
-int prefill_reserve(nda_ctx *c, const PrefillPlan &pl);
+int prefill_reserve(nda_ctx *c, PrefillPlan &pl);
 
 // the front (nda_api_front.hip): initialised, weights present, each
 // sequence at most once, every position inside the rotary table

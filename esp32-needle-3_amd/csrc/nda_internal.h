@@ -75,8 +75,11 @@ struct PrefillArgs {
                                 prefix id (-1: none); GQA decode: [rows] the rows' work order,
                                 or null */
     const uint32_t *row_seq; /* decode launches (one wave per item): sequence of each row, or null */
-    float *part;             /* shared-prefix decode pass: split-KV partials of chunk 0, or null */
-    uint32_t max_chunks;     /*   their stride (AttnArgs::max_chunks) */
+    float *part;             /* shared-prefix decode pass: split-KV partials of chunk 0; split keys:
+                                [T][nh][ksplit][part_stride] states for the merge; or null */
+    uint32_t max_chunks;     /*   parts per (row, head) (AttnArgs::max_chunks; ksplit) */
+    uint32_t part_stride;    /*   floats per part (prefix pass: dv + 2) */
+    uint32_t ksplit;         /* prefill: parts each item's key tiles are split into, 0: not split */
     uint32_t tab_cap;        /* prefill: key tiles of the longest work item (its per-work-group tile
                                 table in LDS), 0: no table */
     PageGeom pg;
@@ -279,6 +282,8 @@ hipError_t launch_prefill(const Geo &g, const PrefillArgs &a, int waves, hipStre
  * size can take (dma: tiles loaded straight into LDS, fp16 at qk 64); a
  * launch whose table would be larger runs without one. */
 uint32_t pf_tab_max_bytes(int waves, bool dma);
+/* The parts of a split-key prefill (a.ksplit: a power of two from 2 to 64) merged into out: units = tokens * nh. */
+hipError_t launch_pf_merge(const PrefillArgs &a, uint64_t units, hipStream_t s);
 /* GQA decode on MFMA: one wave per (row, kv-head) item, n_items = rows * nkv,
  * items in (row, kv-head) order; a.row_seq as in AttnArgs. */
 bool decode_mfma_supported(const Geo &g);

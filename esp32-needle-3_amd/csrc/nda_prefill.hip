@@ -27,6 +27,7 @@
 // :2250-2252).
 #include "nda_device.h"
 
+#include <algorithm>
 #include <float.h>
 
 namespace nda {
@@ -300,13 +301,16 @@ struct PfIO {
     int tid, wave, n_sh, own_len;
     // processing order: full shared tiles [0, nfs), own tiles visible to
     // every row [nfs, jfull), then the masked ones: the partial shared tile
-    // (psh = 1 if there is one), then the own tiles crossing the diagonal
-    int nfs, psh, jfull, ntile;
+    // (psh = 1 if there is one), then the own tiles crossing the diagonal.
+    // This work-group runs the ntile tiles from t0 on (all of them unless
+    // the keys are split); tile indices elsewhere count from t0.
+    int nfs, psh, jfull, t0, ntile;
 
-    // tile t of the processing order: segment, first slot, segment length
-    // (selects, no branches: this runs on the scalar unit every tile)
+    // tile t: segment, first slot, segment length (selects, no branches:
+    // this runs on the scalar unit every tile)
     __device__ __forceinline__ void seg(int t, bool &sh, int &s0, int &len) const
     {
+        t += t0;
         const bool tail = psh != 0 && t == jfull;       // the partial shared tile
         sh = t < nfs || tail;
         const int own = t - nfs - (t > jfull ? psh : 0);
@@ -525,13 +529,36 @@ void prefill_kernel(PrefillArgs a)
     // rows are decode queries of sequences attached to it, packed across
     // them, and it leaves each row's softmax state for the sequences' own
     // positions to continue.
-    const bool partial = a.part != nullptr;
+    // Split keys (a.ksplit parts, blockIdx.y): the work-group attends its
+    // share of the item's tiles and leaves the rows' states for
+    // pf_merge_kernel.
+    const bool partial = a.part != nullptr && a.ksplit == 0;
     io.own_len = partial ? 0 : kmax - n_sh;         // own slots [0, own_len) are touched
     io.nfs = n_sh / PF_KT;
     io.psh = n_sh % PF_KT != 0;
     io.jfull = io.nfs + (partial ? 0 : (kfull - n_sh) / PF_KT);   // + own tiles visible to every row
     io.ntile = io.nfs + io.psh + (io.own_len + PF_KT - 1) / PF_KT;
-    const int ntile = io.ntile, jfull = io.jfull;
+    io.t0 = 0;
+    if (a.ksplit) {
+        const int all = io.ntile, y = (int)blockIdx.y, S = (int)a.ksplit;
+        io.t0 = (int)((int64_t)all * y / S);
+        io.ntile = (int)((int64_t)all * (y + 1) / S) - io.t0;
+        if (io.ntile == 0) {        // more parts than tiles: an empty state
+            // the row from an opaque copy of the thread id: shared with the
+            // tiles' row index it cost the 2-wave DMA variant a spill
+            int te = tid;
+            asm volatile("" : "+v"(te));
+            const int re = r0 + (te >> 6) * 32 + (te & 31);
+            if (re < nrows && (te & 32) == 0) {
+                const uint64_t qr = (uint64_t)(tok0 + re / REP) * a.nh + (int)g * REP + re % REP;
+                float *pr = a.part + (qr * S + y) * a.part_stride + DV;
+                pr[0] = -FLT_MAX;
+                pr[1] = 0.0f;
+            }
+            return;
+        }
+    }
+    const int ntile = io.ntile, jfull = min(max(io.jfull - io.t0, 0), ntile);
 
     // TAB: the tile table (dynamic LDS of a.tab_cap entries, at least every
     // item's tile count), one entry per thread and pass
@@ -913,10 +940,12 @@ void prefill_kernel(PrefillArgs a)
         qrow_e = (uint64_t)(tok0 + re / REP) * a.nh + (int)g * REP + re % REP;
         jh_e = (te >> 5) & 1;
     }
-    if (partial) {
-        // split-KV chunk 0 of the row: unnormalised sums, the running max
-        // (base 2) and the sum of weights, as the decode kernel's partials
-        float *pr = a.part + qrow_e * a.max_chunks * (DV + 2);
+    if (a.part != nullptr) {
+        // the row's state: unnormalised sums, the running max (base 2) and
+        // the sum of weights. A prefix pass: split-KV chunk 0, as the decode
+        // kernel's partials; split keys: part blockIdx.y, rows of 16-byte
+        // multiples for pf_merge_kernel.
+        float *pr = a.part + (qrow_e * a.max_chunks + blockIdx.y) * a.part_stride;
 #pragma unroll
         for (int dt = 0; dt < 2; dt++) {
             const float16v &acc = dt == 0 ? acc0 : acc1;
@@ -953,6 +982,80 @@ void prefill_kernel(PrefillArgs a)
             *reinterpret_cast<float4 *>(o + d0) = z;
         }
     }
+}
+
+// Merge of a split-key prefill: 16 lanes per (token, head), four dims each.
+// Latency bound (4-5 us with the launch): up to 16 parts' loads are issued
+// before any is used. A part that visited no tile left only its empty state
+// (weight sum 0).
+template <int S>
+__global__ __launch_bounds__(256) void pf_merge_kernel(PrefillArgs a, uint64_t units)
+{
+    constexpr int DV = 64;
+    const uint64_t u = (uint64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (u >= units)
+        return;
+    const int d0 = 4 * (int)(threadIdx.x & 15);
+    const float *pr = a.part + u * S * a.part_stride;
+    constexpr int B = S < 16 ? S : 16;
+    float M = -FLT_MAX, L = 0.0f;
+    float4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int s0 = 0; s0 < S; s0 += B, pr += B * a.part_stride) {
+        float2 ml[B];
+        float4 v[B];
+#pragma unroll
+        for (int s = 0; s < B; s++) {
+            ml[s] = *reinterpret_cast<const float2 *>(pr + s * a.part_stride + DV);
+            v[s] = *reinterpret_cast<const float4 *>(pr + s * a.part_stride + d0);
+        }
+        float Mn = M;
+#pragma unroll
+        for (int s = 0; s < B; s++)
+            Mn = __builtin_fmaxf(Mn, ml[s].x);
+        const float r = fast_exp2(M - Mn);
+        M = Mn;
+        L *= r;
+        o.x *= r;
+        o.y *= r;
+        o.z *= r;
+        o.w *= r;
+#pragma unroll
+        for (int s = 0; s < B; s++) {
+            if (ml[s].y == 0.0f)
+                continue;
+            const float w = fast_exp2(ml[s].x - M);
+            L += ml[s].y * w;
+            o.x += v[s].x * w;
+            o.y += v[s].y * w;
+            o.z += v[s].z * w;
+            o.w += v[s].w * w;
+        }
+    }
+    const float inv = 1.0f / L;
+    float4 z = {o.x * inv, o.y * inv, o.z * inv, o.w * inv};
+    if (a.gate) {
+        const float4 g = *reinterpret_cast<const float4 *>(a.gate + u * DV + d0);
+        z.x *= sigmoid_dev(g.x);
+        z.y *= sigmoid_dev(g.y);
+        z.z *= sigmoid_dev(g.z);
+        z.w *= sigmoid_dev(g.w);
+    }
+    *reinterpret_cast<float4 *>(a.out + u * DV + d0) = z;
+}
+
+hipError_t launch_pf_merge(const PrefillArgs &a, uint64_t units, hipStream_t s)
+{
+    if (units == 0)
+        return hipSuccess;
+    const dim3 grid((unsigned)((units + 15) / 16));
+    switch (a.ksplit) {
+#define X(S) case S: hipLaunchKernelGGL((pf_merge_kernel<S>), grid, dim3(256), 0, s, a, units); break;
+    X(2) X(4) X(8) X(16) X(32) X(64)
+#undef X
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 // ------------------------------------------------------------ GQA decode
@@ -1507,7 +1610,8 @@ hipError_t launch_prefill(const Geo &g, const PrefillArgs &a, int waves, hipStre
     if (waves == 8 && !pf_w8_fits(g))
         waves = 4;
     const int es = g.kv_f16 ? 2 : 1;
-    dim3 grid(a.n_items);     // n_items: a multiple of 8 (padded with empty items)
+    // n_items: a multiple of 8 (padded with empty items)
+    dim3 grid(a.n_items, std::max(1u, a.ksplit));
     // a table of a.tab_cap tiles when the host sized one that fits
     const uint32_t tab_bytes = a.tab_cap * 16u;
     const bool tab = a.tab_cap > 0 && tab_bytes <= pf_tab_max_bytes(waves, es == 2 && g.dk == 64 && g.dv == 64);

@@ -757,6 +757,51 @@ def test_prefill_small_groups_direct_and_staged_tiles(hist, ntok):
     assert worst <= TOL, worst
 
 
+# Split-key prefills keep the scores' precision (hi/lo pairs, 2^-22 relative
+# on scores of at most 8 here): weights within 8 log2(e) 2^-21 = 5.5e-6, values
+# of at most 4, so 2.2e-5; a merge adds a few 2^-24.
+SPLIT_TOL = 2.5e-5
+
+
+@pytest.mark.parametrize("kv_dtype,nh,nkv,qk,hist,ntok,gated", [
+    (O.KV_F16, 8, 8, 64, [2500], [40], True),                        # 64-row groups, 32 parts
+    (O.KV_F16, 8, 8, 64, [0, 700, 3, 40], [1, 300, 2, 33], False),   # empty parts, parts above the diagonal
+    (O.KV_INT8, 12, 2, 48, [600, 0], [60, 129], True),               # GQA rows, a chunk's own tiles split
+    (O.KV_INT8, 8, 8, 64, [352], [1], True),                         # the smallest: 12 tiles, one row
+])
+def test_prefill_split_keys(kv_dtype, nh, nkv, qk, hist, ntok, gated):
+    """Launches of few work items split each item's key tiles over several
+    work-groups and merge their states."""
+    say("prefill split keys", kv_dtype, nh, nkv, qk, hist, ntok)
+    worst, _ = _prefill_case(kv_dtype, nh, nkv, qk, hist, ntok, seed=61 + nh, gated=gated)
+    assert worst <= SPLIT_TOL, worst
+
+
+@pytest.mark.parametrize("npre,suffix", [(500, [40, 1]), (512, [33]), (395, [64, 3, 20])])
+def test_prefill_split_keys_shared_prefix(npre, suffix):
+    """The same over a shared prefix, whose partial last tile comes after the
+    full own tiles: split and VALU launches agree."""
+    say("prefill split keys, shared prefix", npre, suffix)
+    N = nda()
+    nh, d, B, outs = 8, 64, len(suffix), []
+    for flags in (0, N.FLAG_PREFILL_VALU):
+        rng = np.random.default_rng(62)
+        ctx = N.Context(1, nh, nh, d, d, 640, kv_dtype=O.KV_F16, max_seqs=B + 1, flags=flags)
+        T = sum(suffix)
+        pre = [N.DevBuf.from_array(rng.standard_normal((npre, nh, d)).astype(np.float32)) for _ in range(3)]
+        ctx.prefill(0, [npre], *pre, N.DevBuf(npre * nh * d * 4), seq_ids=[B])
+        ctx.advance(1, [B], npre)
+        pid = ctx.prefix_build(B)
+        for b in range(B):
+            ctx.seq_attach(b, pid)
+        x = [N.DevBuf.from_array(rng.standard_normal((T, nh, d)).astype(np.float32)) for _ in range(3)]
+        dout = N.DevBuf(T * nh * d * 4)
+        ctx.prefill(0, suffix, *x, dout)
+        ctx.sync()
+        outs.append(dout.to_array(np.float32, (T, nh * d)))
+    assert maxdiff(*outs) <= SPLIT_TOL
+
+
 def test_prefill_mfma_matches_valu_path():
     say("prefill mfma vs valu")
     hist, ntok = [17, 300], [90, 45]
