@@ -407,6 +407,7 @@ AttnArgs attn_args(nda_ctx *c, uint32_t layer, uint32_t rows, const float *q, co
     // grid.y and the partial-buffer stride: chunks of the longest row.
     a.max_chunks = std::max<uint32_t>(1, (max_total + a.chunk - 1) / a.chunk);
     a.qscale = (float)(1.4426950408889634 / std::sqrt((double)c->cfg.qk_head_dim));
+    a.cus = (uint32_t)c->cus;
     a.avg_len = rows ? (uint32_t)std::min<uint64_t>(sum_total / rows, 0xFFFFFFFFu) : 0;
     return a;
 }
@@ -416,11 +417,7 @@ AttnArgs attn_args(nda_ctx *c, uint32_t layer, uint32_t rows, const float *q, co
 // the group's heads as its rows (S^T = K.Q^T, O^T += V^T.P^T), where the
 // VALU kernel spends its time on per-lane dot products and their lane
 // reductions (2.5x on 4096 rows of the engine's 12/2-head shape). Launches
-// that fuse the store, carry per-row offsets or split rows stay on the VALU
-// kernel, and so do tiny ones (an engine session), whose VALU waves split
-// each row's positions between them.
-constexpr uint64_t MFMA_DECODE_MIN_ITEMS = 16;
-
+// that carry per-row offsets or split rows stay on the VALU kernel.
 bool mfma_decode_geo(const nda_ctx *c)
 {
     return decode_mfma_supported(c->geo) && !(c->cfg.flags & NDA_FLAG_DECODE_VALU);
@@ -428,8 +425,22 @@ bool mfma_decode_geo(const nda_ctx *c)
 
 bool mfma_decode(const nda_ctx *c, const AttnArgs &a)
 {
-    return mfma_decode_geo(c) && !a.k_new && !a.row_t && a.max_chunks == 1 &&
-           (uint64_t)a.rows * c->cfg.n_kv_heads >= MFMA_DECODE_MIN_ITEMS;
+    return mfma_decode_geo(c) && !a.row_t && a.max_chunks == 1 && (!a.k_new || mfma_decode_waves(c, a.rows) > 1);
+}
+
+// Waves per (row, kv-head) of the MFMA decode. Where one wave per item
+// leaves the chip idle, a row's tiles are split over several (12/2 heads,
+// rows of 213-383 positions, us): one session 23.9 (the VALU kernel) -> 5.2
+// with 8 waves; 600 items 15.0 with one wave, 9.8 with 4, 13.8 with 8; 1024
+// items 14.1, 10.6, 14.0; 1400 items 15.5, 14.6, 19.4; 2048 items 16.9,
+// 18.6, 26.2. Up to one item per CU 8 waves gain on long rows (16 items of
+// 700-1000 positions 8.6 against 10.6) and lose nothing on short ones.
+// Launches of several waves also fuse a step's store (the one-wave VALU
+// kernel took 40 us for it).
+int mfma_decode_waves(const nda_ctx *c, uint32_t rows)
+{
+    const uint64_t items = (uint64_t)rows * c->cfg.n_kv_heads, cus = (uint64_t)c->cus;
+    return items <= cus ? 8 : items <= 5 * cus ? 4 : 1;
 }
 
 // Device buffers an attention launch over `rows` rows needs: the row staging

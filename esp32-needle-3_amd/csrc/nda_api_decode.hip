@@ -69,11 +69,13 @@ int run_attend(nda_ctx *c, AttnArgs &a, hipStream_t st, float *part, bool prof, 
         pa.n_items = a.rows * c->cfg.n_kv_heads;
         pa.nh = a.nh;
         pa.qscale = a.qscale;
+        pa.k_new = a.k_new;
+        pa.v_new = a.v_new;
         // enough rows for several rounds of waves, rows 0..rows-1
         if (ordered && !a.row_seq && pa.n_items >= 4u * (uint32_t)c->cus)
             pa.items = decode_order(c, a.rows, st);
         ProfScope ps(c, NDA_K_DECODE, st, prof);
-        hipError_t e = launch_decode_mfma(c->geo, pa, st);
+        hipError_t e = launch_decode_mfma(c->geo, pa, mfma_decode_waves(c, a.rows), st);
         if (e != hipSuccess)
             return hip_fail(c, e, "decode (MFMA) kernel launch");
         return NDA_OK;

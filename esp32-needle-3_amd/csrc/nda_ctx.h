@@ -265,6 +265,7 @@ AttnArgs attn_args(nda_ctx *c, uint32_t layer, uint32_t rows, const float *q, co
                    float *out, uint32_t max_total, uint64_t sum_total);
 bool mfma_decode_geo(const nda_ctx *c);
 bool mfma_decode(const nda_ctx *c, const AttnArgs &a);
+int mfma_decode_waves(const nda_ctx *c, uint32_t rows);
 int reserve_attend(nda_ctx *c, uint32_t rows, bool staged, uint32_t max_total, uint64_t sum_total);
 // part: split-KV partials of at least rows * nh * max_chunks * (v_hd + 2)
 // floats, or null for the context's own buffer (grown on demand). prof: record

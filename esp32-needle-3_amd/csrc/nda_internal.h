@@ -58,6 +58,7 @@ struct AttnArgs {
     const float *k_new;      /* [rows][nkv][dk] fused append (decode), or null */
     const float *v_new;      /* [rows][nkv][dv] */
     uint32_t avg_len;        /* mean visible positions per row (work-group size) */
+    uint32_t cus;            /* compute units (work-group size) */
 };
 
 /* One launch of the MFMA causal-prefill kernel. A work item is one tile of
@@ -86,6 +87,8 @@ struct PrefillArgs {
     uint32_t n_items;
     uint32_t nh;
     float qscale;
+    const float *k_new;      /* decode launches of several waves per item: the new rows to store first */
+    const float *v_new;      /*   ([rows][nkv][dk], [rows][nkv][dv]), or null */
 };
 
 struct AppendArgs {
@@ -284,10 +287,11 @@ hipError_t launch_prefill(const Geo &g, const PrefillArgs &a, int waves, hipStre
 uint32_t pf_tab_max_bytes(int waves, bool dma);
 /* The parts of a split-key prefill (a.ksplit: a power of two from 2 to 64) merged into out: units = tokens * nh. */
 hipError_t launch_pf_merge(const PrefillArgs &a, uint64_t units, hipStream_t s);
-/* GQA decode on MFMA: one wave per (row, kv-head) item, n_items = rows * nkv,
- * items in (row, kv-head) order; a.row_seq as in AttnArgs. */
+/* GQA decode on MFMA: `waves` waves (1, 4 or 8) per (row, kv-head) item,
+ * n_items = rows * nkv, items in (row, kv-head) order; a.row_seq as in
+ * AttnArgs. */
 bool decode_mfma_supported(const Geo &g);
-hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, hipStream_t s);
+hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, int waves, hipStream_t s);
 hipError_t launch_combine(const Geo &g, const AttnArgs &a, hipStream_t s);
 hipError_t launch_copy(const Geo &g, const CopyArgs &a, hipStream_t s);
 hipError_t launch_gather(const Geo &g, const StageArgs &a, hipStream_t s);

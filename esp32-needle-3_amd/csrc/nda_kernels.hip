@@ -851,7 +851,8 @@ __global__ __launch_bounds__(256) void fill_kv_kernel(FillKvArgs a)
 template <int ES, int DK, int REP>
 constexpr int lanes_per_pos() { return ES == 2 ? 8 : ((REP >= 8 && DK % 64 == 0) ? 8 : 4); }
 
-// Waves per decode work-group. Wide GQA (rep >= 4): one, since each lane
+// Waves per decode work-group where there are items enough (att_few is the
+// rule for the others). Wide GQA (rep >= 4): one, since each lane
 // carries rep heads of state and the cross-wave merge would cost more than
 // it parallelises (rows of a few hundred positions: 4.4x faster at 12 q /
 // 2 kv heads, int8). MHA and narrow GQA: eight for work items of 448
@@ -870,6 +871,28 @@ constexpr int att_nw(bool long_items)
 #endif
 }
 constexpr uint32_t ATT_LONG_ITEM = 448;
+
+// Launches of few work items are bound by one work-group's walk along its
+// positions, whatever the geometry, so those of long enough rows run eight
+// waves (us, before -> now):
+//   - rep >= 4 (one wave elsewhere), up to 3 items per CU of 128 positions or
+//     more: 12/2 heads fp16, 213-383 positions, 1 sequence 24 -> 15, 32 36.5
+//     -> 17.8, 256 55 -> 28, 400 58 -> 46 (at 90 positions 240 sequences
+//     19.7 -> 21.8); in chunks of 1024 of 4-8K positions, 2 sequences fp16 90
+//     -> 26, int8 62 -> 30, 32 sequences 136 -> 43 and 85 -> 66;
+//   - rep <= 2 (two waves elsewhere), up to 2 items per CU: 8 heads, 213-383
+//     positions, 64 sequences fp16 22 -> 12, int8 14.7 -> 11.6 (96 sequences
+//     int8 16.8 -> 19.0); at 180 positions 60 sequences fp16 13.5 -> 9.3, but
+//     4 sequences int8 7.3 -> 8.0: the merge of eight states costs about 1 us.
+constexpr int ATT_FEW_NW = 8;
+template <int ES, int REP>
+static bool att_few(const AttnArgs &a)
+{
+    const uint64_t items = (uint64_t)a.rows * a.pg.nkv * (a.max_chunks - a.chunk_lo);
+    const uint32_t len = a.avg_len < a.chunk ? a.avg_len : a.chunk;
+    return a.chunk_lo == 0 && items <= (REP >= 4 ? 3ull : 2ull) * a.cus &&
+           len >= (REP >= 4 ? 128u : ES == 2 ? 160u : 256u);
+}
 
 // Positions per lane group per step. fp16 at rep <= 2: 4 (80 registers, 6
 // waves per SIMD); 8 also fits without spilling (120 registers) but leaves 4
@@ -940,7 +963,12 @@ static void launch_attend_hs(const AttnArgs &a, hipStream_t s)
 template <int ES, int DK, int DV, int REP, bool RT>
 static void launch_attend_geo(const AttnArgs &a, bool long_items, hipStream_t s)
 {
-    if (att_hs<REP>() > 1 && !a.k_new)
+    if (att_few<ES, REP>(a)) {
+        if (att_hs<REP>() > 1 && !a.k_new)
+            launch_attend_hs<ES, DK, DV, REP, att_hs<REP>(), ATT_FEW_NW, RT>(a, s);
+        else
+            launch_attend_hs<ES, DK, DV, REP, 1, ATT_FEW_NW, RT>(a, s);
+    } else if (att_hs<REP>() > 1 && !a.k_new)
         launch_attend_hs<ES, DK, DV, REP, att_hs<REP>(), 1, RT>(a, s);
     else if (long_items)
         launch_attend_hs<ES, DK, DV, REP, 1, att_nw<REP>(true), RT>(a, s);

@@ -1112,15 +1112,22 @@ __device__ __forceinline__ float4v mfma16k32(half8 a, half8 b, float4v c)
 // read slots of the same pages (or half 0 again) and are masked.
 //
 // A wave keeps one tile in flight in registers (loaded while the previous
-// one is computed) and one in its LDS buffer. Splitting a row's tiles over
-// more waves (and merging their states) measured no faster: the launch is
-// bound by its memory stream, not by the wave count.
+// one is computed) and one in its LDS buffer.
+//
+// NW: waves per (row, kv-head). A launch that fills the chip runs one: it is
+// bound by its memory stream, and more waves per row measured no faster. A
+// launch of few rows is bound by one wave's chain of about 1 us per tile
+// instead (24 sequences of 213-383 positions: 14.2 us with one wave, 7.2
+// with eight; one session 23.9 us on the VALU kernel, 5.2 here), so its
+// work-groups split a row's tiles over NW waves, each with its own buffer and
+// softmax state, which meet in LDS at the end. Such a launch may also store
+// the new row first (a.k_new, as the VALU kernel's fused append).
 //
 // RUN (pages of 16 slots, K + V + scales of a kv-head within 128 chunks of
 // 16 bytes): a half tile is a whole kv-head block of one page, 1920 bytes at
 // qk 48, read as one contiguous run by two loads.
-template <int DK, int DV, int REP, bool RUN>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+template <int DK, int DV, int REP, bool RUN, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)))
 void decode_mfma_kernel(PrefillArgs a)
 {
     static_assert(DK % 16 == 0 && DK <= 64 && DV == 64 && REP <= 16,
@@ -1136,9 +1143,14 @@ void decode_mfma_kernel(PrefillArgs a)
     constexpr bool TAIL = DK % 32 == 16;
     constexpr int VSTR = DV + 16;               // V row stride: spreads the transposed reads over the banks
     constexpr int KB = PF_KT * DK, VB = PF_KT * VSTR;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[KB + VB + PF_KT * 8];   // K, V, k scales, v scales
+    // K, V, k scales, v scales of a wave's tile; with several waves, the
+    // merge's states (four float4 and (max, weight sum) per lane) after them
+    constexpr int WB = NW == 1 ? KB + VB + PF_KT * 8 : (KB + VB + PF_KT * 8 > 64 * 72 ? KB + VB + PF_KT * 8 : 64 * 72);
+    __shared__ __attribute__((aligned(16))) uint8_t lds_all[NW * WB];
 
-    const int lane = threadIdx.x;
+    const int lane = NW == 1 ? threadIdx.x : threadIdx.x & 63;
+    const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint8_t *const lds = lds_all + wave * WB;
     const int g = lane >> 4, r = lane & 15;     // MFMA: lane group, row / column
     const uint32_t nkv = a.pg.nkv;
     // a.items: the rows' work order (longest first), or null: in order
@@ -1207,7 +1219,9 @@ void decode_mfma_kernel(PrefillArgs a)
     const cptr own = (cptr)(a.page_table + (uint64_t)seq * a.pg.pages_per_seq);
     const cptr pre = sd.prefix >= 0 ? (cptr)(a.prefix_pages + (uint64_t)sd.prefix * a.pg.pages_per_seq) : own;
     const int tiles_sh = (n_sh + PF_KT - 1) / PF_KT;
-    const int ntile = tiles_sh + (n_own + PF_KT - 1) / PF_KT;
+    const int tiles = tiles_sh + (n_own + PF_KT - 1) / PF_KT;
+    // this wave's tiles [tile0, ntile); with more waves than tiles some have none
+    const int tile0 = NW == 1 ? 0 : tiles * wave / NW, ntile = NW == 1 ? tiles : tiles * (wave + 1) / NW;
     // tile j: its segment's visible slots from its first on
     auto remaining = [&](int j) __attribute__((always_inline)) {
         return j < tiles_sh ? n_sh - PF_KT * j : n_own - PF_KT * (j - tiles_sh);
@@ -1219,7 +1233,7 @@ void decode_mfma_kernel(PrefillArgs a)
         int sip[2], vis[2];                     // vis: the half's visible slots (RUN)
     };
     auto fetch = [&](int j, TileRef &tr_) __attribute__((always_inline)) {
-        j = min(j, ntile - 1);
+        j = NW == 1 ? min(j, ntile - 1) : min(j, max(ntile - 1, tile0));
         const bool sh = j < tiles_sh;
         const int s0 = PF_KT * (sh ? j : j - tiles_sh);
         const int len = sh ? n_sh : n_own;
@@ -1268,55 +1282,74 @@ void decode_mfma_kernel(PrefillArgs a)
         }
     };
 
+    if (NW > 1 && a.k_new) {
+        // the new position's row, before any wave reads its slot: one CU's
+        // L1 serves them all, so the barrier is all the visibility needed
+        if (wave == 0) {
+            const int slot = own_slot(sd, sd.pos, (int)a.pg.window);
+            const int32_t page = own[slot >> a.pg.log2_page];
+            if (page >= 0) {
+                uint8_t *hb = const_cast<uint8_t *>(a.pool) + (uint64_t)page * a.pg.page_bytes + (uint64_t)kvh * a.pg.head_bytes;
+                const float kx = lane < DK ? a.k_new[((uint64_t)b * nkv + kvh) * DK + lane] : 0.0f;
+                const float vx = lane < DV ? a.v_new[((uint64_t)b * nkv + kvh) * DV + lane] : 0.0f;
+                store_row<1>(hb, slot & (P - 1), P, kx, vx, lane, DK, DV);
+            }
+        }
+        __syncthreads();
+    }
+
     // the first tile goes out before the q loads, so that their latencies
     // overlap; tref then holds the references of the next tile
     TileRef tref;
     Stage sg;
-    fetch(0, tref);
+    fetch(tile0, tref);
     load(tref, sg);
-    fetch(1, tref);
+    fetch(tile0 + 1, tref);
 
     // Q^T operand, hi and lo: column r, dims 32 s + 8 g + [0, 8) and the tail
     // 32 NS + 4 g + [0, 4) (then four zero slots); hi and lo from one rounded
-    // fp32 value
+    // fp32 value. Several waves: of the column's q * 2^qexp, whose largest
+    // is in [2^14, 2^15) (see the weights in the tile).
     const bool rvalid = r < REP;
     const uint64_t qrow = (uint64_t)b * a.nh + kvh * REP + (rvalid ? r : 0);
     half8 qh[NS + TAIL], ql[NS + TAIL];
+    int qexp = 0;
     {
         const float *qr = a.q + qrow * DK;
         const float qs = rvalid ? a.qscale : 0.0f;
-        auto split = [&](float v, _Float16 &hi, _Float16 &lo) __attribute__((always_inline)) {
-            float x = v * qs;
-            asm volatile("" : "+v"(x));
-            hi = (_Float16)x;
-            lo = (_Float16)(x - (float)hi);
-        };
+        float x[NS + TAIL][8];
 #pragma unroll
-        for (int st = 0; st < NS; st++) {
-            const float4 v0 = *reinterpret_cast<const float4 *>(qr + 32 * st + 8 * g);
-            const float4 v1 = *reinterpret_cast<const float4 *>(qr + 32 * st + 8 * g + 4);
+        for (int st = 0; st < NS + TAIL; st++) {
+            const bool tail = st == NS;
+            const float4 v0 = *reinterpret_cast<const float4 *>(qr + 32 * st + (tail ? 4 : 8) * g);
+            const float4 v1 = tail ? float4{0.0f, 0.0f, 0.0f, 0.0f}
+                                   : *reinterpret_cast<const float4 *>(qr + 32 * st + 8 * g + 4);
             const float xs[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                _Float16 hi, lo;
-                split(xs[i], hi, lo);
-                qh[st][i] = hi;
-                ql[st][i] = lo;
-            }
+            for (int i = 0; i < 8; i++)
+                x[st][i] = xs[i] * qs;
         }
-        if constexpr (TAIL) {
-            const float4 v = *reinterpret_cast<const float4 *>(qr + 32 * NS + 4 * g);
-            const float xs[4] = {v.x, v.y, v.z, v.w};
-            qh[NS] = half8{};
-            ql[NS] = half8{};
+        if constexpr (NW > 1) {
+            float mx = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                _Float16 hi, lo;
-                split(xs[i], hi, lo);
-                qh[NS][i] = hi;
-                ql[NS][i] = lo;
-            }
+            for (int st = 0; st < NS + TAIL; st++)
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    mx = fmaxf(mx, fabsf(x[st][i]));
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            if (mx > 0.0f && mx <= FLT_MAX)
+                qexp = 15 - __builtin_amdgcn_frexp_expf(mx);
         }
+#pragma unroll
+        for (int st = 0; st < NS + TAIL; st++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                float v = NW > 1 ? ldexpf(x[st][i], qexp) : x[st][i];
+                asm volatile("" : "+v"(v));
+                qh[st][i] = (_Float16)v;
+                ql[st][i] = (_Float16)(v - (float)qh[st][i]);
+            }
     }
 
     // lane-constant LDS offsets: the S operand rows (block 0; block 1 is 4
@@ -1328,12 +1361,16 @@ void decode_mfma_kernel(PrefillArgs a)
 
     float4v acc[4] = {};                        // O^T: dims 16 d + 4 g + i, column r
     float m = -FLT_MAX, lsum = 0.0f;
+    int vexp = 0;                               // several waves: acc counts in 2^(vexp - 7) (see the tile)
     const float neg1 = opaque_neg1();
 
     // the gate of this lane's output dims 16 d + 4 g + [0, 4), loaded with
     // the last tile's arithmetic, so that its latency does not end the wave
+    // (several waves: wave d emits dims 16 d + 4 g + [0, 4))
     const float *gt = a.gate ? a.gate + qrow * DV : nullptr;
     float4 gv4[4];
+    if (NW > 1 && gt && wave < 4)
+        gv4[0] = *reinterpret_cast<const float4 *>(gt + 16 * wave + 4 * g);
 
     // tile j: the load of the next tile (references fetched a tile ago), the
     // references of the one after, the tile's arithmetic, then the next tile
@@ -1348,7 +1385,7 @@ void decode_mfma_kernel(PrefillArgs a)
         if constexpr (more) {
             load(tref, sg);
             fetch(j + 2, tref);
-        } else {
+        } else if constexpr (NW == 1) {
 #pragma unroll
             for (int d = 0; d < 4; d++)
                 gv4[d] = gt && rvalid ? *reinterpret_cast<const float4 *>(gt + 16 * d + 4 * g) : float4{0, 0, 0, 0};
@@ -1380,7 +1417,9 @@ void decode_mfma_kernel(PrefillArgs a)
         const float nm = -m;
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
-            const float4 ks = *reinterpret_cast<const float4 *>(lds + soff + 16 * kb);
+            float4 ks = *reinterpret_cast<const float4 *>(lds + soff + 16 * kb);
+            if constexpr (NW > 1)
+                ks = float4{ldexpf(ks.x, -qexp), ldexpf(ks.y, -qexp), ldexpf(ks.z, -qexp), ldexpf(ks.w, -qexp)};
             const float4 vs = *reinterpret_cast<const float4 *>(lds + soff + 128 + 16 * kb);
             if constexpr (FIRST) {
                 st[kb] *= float4v{ks.x, ks.y, ks.z, ks.w};
@@ -1416,10 +1455,10 @@ void decode_mfma_kernel(PrefillArgs a)
         }
         if constexpr (FIRST) {
             // the first tile sets m (nothing is accumulated yet)
-            m = mt;
+            m = NW == 1 ? mt : __builtin_fmaxf(mt, -FLT_MAX);
 #pragma unroll
             for (int kb = 0; kb < 2; kb++)
-                st[kb] -= mt;
+                st[kb] -= m;
         } else {
             // scores relative to m: it moves only when one exceeds it by 2^8
             const bool grow = mt > 8.0f;
@@ -1436,6 +1475,29 @@ void decode_mfma_kernel(PrefillArgs a)
                     st[kb] -= d;
             }
         }
+        if constexpr (NW > 1) {
+            // These launches took over from fp32 products, whose accuracy
+            // the fp16 pairs reach if no lo half is subnormal and hi is
+            // rounded to nearest: the v scales (about 0.02) are brought to
+            // 2^7 by a power of two that follows the largest seen, as m
+            // follows the scores.
+            float vm = max3(max3(vsc[0], vsc[1], vsc[2]), max3(vsc[3], vsc[4], vsc[5]), max3(vsc[6], vsc[7], vsc[7]));
+            vm = max3(vm, __shfl_xor(vm, 16, 64), vm);
+            vm = max3(vm, __shfl_xor(vm, 32, 64), vm);
+            const int ve = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_expf(vm));
+            if (FIRST || ve > vexp) {
+                if constexpr (!FIRST)
+#pragma unroll
+                    for (int d = 0; d < 4; d++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+                            acc[d][i] = ldexpf(acc[d][i], vexp - ve);
+                vexp = ve;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                vsc[i] = ldexpf(vsc[i], 7 - vexp);      // weight * scale < 2^8 * 2^7
+        }
         float p[8];
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
@@ -1447,12 +1509,19 @@ void decode_mfma_kernel(PrefillArgs a)
         for (int i = 0; i < 8; i++)
             p[i] *= vsc[i];
         // P^T operand (hi, lo): slots = keys 8 g .. 8 g + 7; hi = p rounded
-        // toward zero to fp16, lo = the remainder
+        // toward zero (several waves: to nearest) to fp16, lo = the remainder
         u32x4 phw, plw;
 #pragma unroll
         for (int i = 0; i < 8; i += 2) {
-            const fp16x2 hh = __builtin_amdgcn_cvt_pkrtz(p[i], p[i + 1]);
-            const uint32_t hw = __builtin_bit_cast(uint32_t, hh);
+            uint32_t hw;
+            if constexpr (NW > 1) {
+                // (lo from this very hi: without the asm the compiler may
+                // round one of them from the exact product)
+                asm volatile("" : "+v"(p[i]), "+v"(p[i + 1]));
+                hw = __builtin_bit_cast(uint32_t, half2v{(_Float16)p[i], (_Float16)p[i + 1]});
+            } else {
+                hw = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p[i], p[i + 1]));
+            }
             phw[i >> 1] = hw;
             plw[i >> 1] = split_lo2(hw, p[i], p[i + 1], neg1);
         }
@@ -1481,17 +1550,17 @@ void decode_mfma_kernel(PrefillArgs a)
     store(sg);
     using Yes = std::true_type;
     using No = std::false_type;
-    if (ntile == 1) {
-        if (remaining(0) >= PF_KT)
-            tile(0, No{}, Yes{}, Yes{});
+    if (ntile - tile0 == 1) {
+        if (remaining(tile0) >= PF_KT)
+            tile(tile0, No{}, Yes{}, Yes{});
         else
-            tile(0, Yes{}, Yes{}, Yes{});
-    } else {
-        if (remaining(0) >= PF_KT)
-            tile(0, No{}, No{}, Yes{});
+            tile(tile0, Yes{}, Yes{}, Yes{});
+    } else if (NW == 1 || tile0 < ntile) {
+        if (remaining(tile0) >= PF_KT)
+            tile(tile0, No{}, No{}, Yes{});
         else
-            tile(0, Yes{}, No{}, Yes{});
-        for (int j = 1; j + 1 < ntile; j++) {
+            tile(tile0, Yes{}, No{}, Yes{});
+        for (int j = tile0 + 1; j + 1 < ntile; j++) {
             if (remaining(j) >= PF_KT)
                 tile(j, No{}, No{}, No{});
             else
@@ -1505,10 +1574,56 @@ void decode_mfma_kernel(PrefillArgs a)
 
     lsum += __shfl_xor(lsum, 16, 64);
     lsum += __shfl_xor(lsum, 32, 64);
+    float *o = a.out + qrow * DV;
+    if constexpr (NW > 1) {
+        // the waves' states into LDS (over the tile buffers), then wave d
+        // merges and emits dims 16 d + 4 g + [0, 4). A wave without tiles
+        // left max -FLT_MAX and zero sums: its weight is 0.
+        // (A wave's own LDS accesses complete in order.)
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                acc[d][i] = ldexpf(acc[d][i], vexp - 7);
+            *reinterpret_cast<float4v *>(lds + 16 * (64 * d + lane)) = acc[d];
+        }
+        *reinterpret_cast<float2 *>(lds + 4096 + 8 * lane) = float2{m, lsum};
+        __syncthreads();
+        if (wave >= 4 || !rvalid)
+            return;
+        float2 ml[NW];
+        float4v av[NW];
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            ml[w] = *reinterpret_cast<const float2 *>(lds_all + w * WB + 4096 + 8 * lane);
+            av[w] = *reinterpret_cast<const float4v *>(lds_all + w * WB + 16 * (64 * wave + lane));
+        }
+        float M = ml[0].x;
+#pragma unroll
+        for (int w = 1; w < NW; w++)
+            M = __builtin_fmaxf(M, ml[w].x);
+        float L = 0.0f;
+        float4v z = {};
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float c = fast_exp2(ml[w].x - M);
+            L += ml[w].y * c;
+            z += av[w] * c;
+        }
+        z *= 1.0f / L;
+        if (gt) {
+            z[0] *= sigmoid_dev(gv4[0].x);
+            z[1] *= sigmoid_dev(gv4[0].y);
+            z[2] *= sigmoid_dev(gv4[0].z);
+            z[3] *= sigmoid_dev(gv4[0].w);
+        }
+        *reinterpret_cast<float4v *>(o + 16 * wave + 4 * g) = z;
+        return;
+    }
     if (!rvalid)
         return;
     const float inv = 1.0f / lsum;
-    float *o = a.out + qrow * DV;
 #pragma unroll
     for (int d = 0; d < 4; d++) {
         const int d0 = 16 * d + 4 * g;
@@ -1541,19 +1656,31 @@ bool decode_mfma_supported(const Geo &g)
     return false;
 }
 
-hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, hipStream_t s)
+template <int DK, int DV, int REP, bool RUN>
+static void launch_dec(const PrefillArgs &a, int waves, hipStream_t s)
+{
+    if (waves == 8)
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 8>), dim3(a.n_items), dim3(512), 0, s, a);
+    else if (waves == 4)
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 4>), dim3(a.n_items), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 1>), dim3(a.n_items), dim3(64), 0, s, a);
+}
+
+hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, int waves, hipStream_t s)
 {
     if (a.n_items == 0)
         return hipSuccess;
+    if (a.k_new && waves == 1)
+        return hipErrorInvalidValue;        // only the several-wave variants store
     const bool p16 = a.pg.log2_page == 4;
-#define X(DK, DV, REP)                                                                                  \
-    if (!g.kv_f16 && g.dk == DK && g.dv == DV && g.rep == REP) {                                        \
-        if (p16 && DK + DV + 8 <= 128)                                                                  \
-            hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, (DK + DV + 8 <= 128)>), dim3(a.n_items), \
-                               dim3(64), 0, s, a);                                                      \
-        else                                                                                            \
-            hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, false>), dim3(a.n_items), dim3(64), 0, s, a); \
-        return hipGetLastError();                                                                       \
+#define X(DK, DV, REP)                                                  \
+    if (!g.kv_f16 && g.dk == DK && g.dv == DV && g.rep == REP) {        \
+        if (p16)                                                        \
+            launch_dec<DK, DV, REP, (DK + DV + 8 <= 128)>(a, waves, s); \
+        else                                                            \
+            launch_dec<DK, DV, REP, false>(a, waves, s);                \
+        return hipGetLastError();                                       \
     }
     NDA_DEC_GEOMETRIES(X)
 #undef X
