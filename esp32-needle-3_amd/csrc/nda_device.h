@@ -71,6 +71,33 @@ __device__ __forceinline__ float xor_lanes(float v, int lane)
     return __builtin_bit_cast(float, r);
 }
 
+// -1.0f that the optimiser cannot see through (one SGPR per kernel, so it
+// costs no VGPR): with it, fma(hi, neg1, p) stays an fma over a widened fp16
+// operand and is selected as one v_fma_mixlo/mixhi_f16 per value; with a
+// literal -1 it is folded into a subtraction and costs a conversion, a
+// subtraction and a packing.
+__device__ __forceinline__ float opaque_neg1()
+{
+    float n = -1.0f;
+    asm volatile("" : "+s"(n));
+    return n;
+}
+
+// lo halves of a pair of values (softmax weights, operands) whose hi halves
+// (rounded to fp16, either way) are packed in hw: fp16(p - hi), rounded to
+// nearest. p - hi is exact in fp32, so the one rounding is the conversion to
+// fp16.
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t split_lo2(uint32_t hw, float p0, float p1, float neg1)
+{
+    const half2v h = __builtin_bit_cast(half2v, hw);
+    half2v l;
+    l[0] = (_Float16)__builtin_fmaf((float)h[0], neg1, p0);
+    l[1] = (_Float16)__builtin_fmaf((float)h[1], neg1, p1);
+    return __builtin_bit_cast(uint32_t, l);
+}
+
 __device__ __forceinline__ int lane_id()
 {
     return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));

@@ -51,32 +51,6 @@ __device__ __forceinline__ float max3(float a, float b, float c)
     return __builtin_fmaxf(__builtin_fmaxf(a, b), c);
 }
 
-// -1.0f that the optimiser cannot see through (one SGPR per kernel, so it
-// costs no VGPR): with it, fma(hi, neg1, p) stays an fma over a widened fp16
-// operand and is selected as one v_fma_mixlo/mixhi_f16 per value; with a
-// literal -1 it is folded into a subtraction and costs a conversion, a
-// subtraction and a packing.
-__device__ __forceinline__ float opaque_neg1()
-{
-    float n = -1.0f;
-    asm volatile("" : "+s"(n));
-    return n;
-}
-
-// lo halves of a pair of softmax weights whose hi halves (rounded toward zero
-// to fp16) are packed in hw: fp16(p - hi), rounded to nearest. p - hi is
-// exact in fp32, so the one rounding is the conversion to fp16.
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t split_lo2(uint32_t hw, float p0, float p1, float neg1)
-{
-    const half2v h = __builtin_bit_cast(half2v, hw);
-    half2v l;
-    l[0] = (_Float16)__builtin_fmaf((float)h[0], neg1, p0);
-    l[1] = (_Float16)__builtin_fmaf((float)h[1], neg1, p1);
-    return __builtin_bit_cast(uint32_t, l);
-}
-
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4v lds_short4v;
 
@@ -1127,13 +1101,17 @@ __device__ __forceinline__ float4v mfma16k32(half8 a, half8 b, float4v c)
 // 16 bytes): a half tile is a whole kv-head block of one page, 1920 bytes at
 // qk 48, read as one contiguous run by two loads.
 template <int DK, int DV, int REP, bool RUN, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW >= 8 ? 2 : 4)))
 void decode_mfma_kernel(PrefillArgs a)
 {
     static_assert(DK % 16 == 0 && DK <= 64 && DV == 64 && REP <= 16,
                   "decode tiles: dk multiple of 16 up to 64, dv 64, rep <= 16");
     static_assert(!RUN || DK + DV + 8 <= 128, "a kv-head block of a 16-slot page within two loads");
     constexpr int NS = DK / 32;                 // 32-dim steps of S (16x16x32)
+    // Eight waves (the smallest launches, two waves per SIMD at most): a
+    // third fp16 part holds what hi and lo leave of an fp32 value, so the
+    // products' operands are exact
+    constexpr bool EXACT = NW >= 8;
     // A last 16-dim step (qk 48) runs on the same 16x16x32 instruction, its
     // upper four k slots zero in both operands. Every accumulation chain
     // thus keeps one opcode: an MFMA reading as its accumulator the result
@@ -1312,7 +1290,7 @@ void decode_mfma_kernel(PrefillArgs a)
     // is in [2^14, 2^15) (see the weights in the tile).
     const bool rvalid = r < REP;
     const uint64_t qrow = (uint64_t)b * a.nh + kvh * REP + (rvalid ? r : 0);
-    half8 qh[NS + TAIL], ql[NS + TAIL];
+    half8 qh[NS + TAIL], ql[NS + TAIL], qx[EXACT ? NS + TAIL : 1];
     int qexp = 0;
     {
         const float *qr = a.q + qrow * DK;
@@ -1348,7 +1326,10 @@ void decode_mfma_kernel(PrefillArgs a)
                 float v = NW > 1 ? ldexpf(x[st][i], qexp) : x[st][i];
                 asm volatile("" : "+v"(v));
                 qh[st][i] = (_Float16)v;
-                ql[st][i] = (_Float16)(v - (float)qh[st][i]);
+                const float l = v - (float)qh[st][i];
+                ql[st][i] = (_Float16)l;
+                if constexpr (EXACT)
+                    qx[st][i] = (_Float16)(l - (float)ql[st][i]);
             }
     }
 
@@ -1397,16 +1378,30 @@ void decode_mfma_kernel(PrefillArgs a)
         for (int kb = 0; kb < 2; kb++) {
             const uint8_t *kr = lds + koff + kb * 4 * DK;
             st[kb] = float4v{};
+            half8 ka[NS + TAIL];
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                const half8 ka = codes8(*reinterpret_cast<const u32x2 *>(kr + 32 * s + 8 * g));
-                st[kb] = mfma16k32(ka, qh[s], st[kb]);
-                st[kb] = mfma16k32(ka, ql[s], st[kb]);
-            }
-            if constexpr (TAIL) {
-                const half8 ka = codes4(*reinterpret_cast<const uint32_t *>(kr + 32 * NS + 4 * g));
-                st[kb] = mfma16k32(ka, qh[NS], st[kb]);
-                st[kb] = mfma16k32(ka, ql[NS], st[kb]);
+            for (int s = 0; s < NS; s++)
+                ka[s] = codes8(*reinterpret_cast<const u32x2 *>(kr + 32 * s + 8 * g));
+            if constexpr (TAIL)
+                ka[NS] = codes4(*reinterpret_cast<const uint32_t *>(kr + 32 * NS + 4 * g));
+            if constexpr (NW == 1) {
+#pragma unroll
+                for (int s = 0; s < NS + TAIL; s++) {
+                    st[kb] = mfma16k32(ka[s], qh[s], st[kb]);
+                    st[kb] = mfma16k32(ka[s], ql[s], st[kb]);
+                }
+            } else {
+                // the small terms first: only the hi products then round at
+                // the score's magnitude
+#pragma unroll
+                for (int s = 0; s < NS + TAIL && EXACT; s++)
+                    st[kb] = mfma16k32(ka[s], qx[s], st[kb]);
+#pragma unroll
+                for (int s = 0; s < NS + TAIL; s++)
+                    st[kb] = mfma16k32(ka[s], ql[s], st[kb]);
+#pragma unroll
+                for (int s = 0; s < NS + TAIL; s++)
+                    st[kb] = mfma16k32(ka[s], qh[s], st[kb]);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1510,7 +1505,7 @@ void decode_mfma_kernel(PrefillArgs a)
             p[i] *= vsc[i];
         // P^T operand (hi, lo): slots = keys 8 g .. 8 g + 7; hi = p rounded
         // toward zero (several waves: to nearest) to fp16, lo = the remainder
-        u32x4 phw, plw;
+        u32x4 phw, plw, pxw;
 #pragma unroll
         for (int i = 0; i < 8; i += 2) {
             uint32_t hw;
@@ -1524,6 +1519,10 @@ void decode_mfma_kernel(PrefillArgs a)
             }
             phw[i >> 1] = hw;
             plw[i >> 1] = split_lo2(hw, p[i], p[i + 1], neg1);
+            if constexpr (EXACT) {
+                const half2v h = __builtin_bit_cast(half2v, hw);
+                pxw[i >> 1] = split_lo2(plw[i >> 1], p[i] - (float)h[0], p[i + 1] - (float)h[1], neg1);
+            }
         }
         const half8 ph = __builtin_bit_cast(half8, phw), pl = __builtin_bit_cast(half8, plw);
         __builtin_amdgcn_sched_barrier(0);
@@ -1532,8 +1531,15 @@ void decode_mfma_kernel(PrefillArgs a)
             const v2i w = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
                 (lds_v2i *)(__attribute__((address_space(3))) void *)(lds + voff + 16 * d));
             const half8 va = codes8(u32x2{(uint32_t)w.x, (uint32_t)w.y});
-            acc[d] = mfma16k32(va, ph, acc[d]);
-            acc[d] = mfma16k32(va, pl, acc[d]);
+            if constexpr (EXACT)
+                acc[d] = mfma16k32(va, __builtin_bit_cast(half8, pxw), acc[d]);
+            if constexpr (NW == 1) {
+                acc[d] = mfma16k32(va, ph, acc[d]);
+                acc[d] = mfma16k32(va, pl, acc[d]);
+            } else {
+                acc[d] = mfma16k32(va, pl, acc[d]);
+                acc[d] = mfma16k32(va, ph, acc[d]);
+            }
         }
         __builtin_amdgcn_s_setprio(0);
         // The next tile into LDS after this tile's last LDS reads. Other lanes
