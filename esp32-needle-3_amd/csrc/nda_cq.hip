@@ -502,6 +502,37 @@ __global__ __launch_bounds__(256) void cq_split_tables_kernel(CqTabArgs a)
         }
 }
 
+// The tensor of a launch's output tile: compares with every bound at once
+// (a walk along them is a chain of scalar loads at the head of every wave).
+__device__ __forceinline__ uint32_t tensor_of(const uint32_t (&tile0)[CQ_MAX_T + 1], uint32_t nt, uint32_t tile)
+{
+    uint32_t b[CQ_MAX_T], t = 0;
+#pragma unroll
+    for (uint32_t k = 1; k < (uint32_t)CQ_MAX_T; k++)
+        b[k] = k < nt ? tile0[k] : 0xFFFFFFFFu;
+#pragma unroll
+    for (uint32_t k = 1; k < (uint32_t)CQ_MAX_T; k++)
+        t = tile >= b[k] ? k : t;
+    return __builtin_amdgcn_readfirstlane(t);
+}
+
+// The eight weights of a lane's k-block as the fp16 pair (wa, wb): tb the
+// column's byte tables, cw the step's codes with the k-block's at bits 0..3
+// of each byte.
+__device__ __forceinline__ void cq_decode8(const uint4 &tb, uint32_t cw, half8 &wa, half8 &wb)
+{
+    const uint32_t b0 = cw & 0x03030303u, h0 = b0 | 0x04040404u;
+    const uint32_t b1 = (cw >> 2) & 0x03030303u, h1 = b1 | 0x04040404u;
+    const uint4 sl = {__builtin_amdgcn_perm(h0, b0, 0x05010400u), __builtin_amdgcn_perm(h0, b0, 0x07030602u),
+                      __builtin_amdgcn_perm(h1, b1, 0x05010400u), __builtin_amdgcn_perm(h1, b1, 0x07030602u)};
+    const u32x4 ua = {__builtin_amdgcn_perm(tb.x, tb.y, sl.x), __builtin_amdgcn_perm(tb.x, tb.y, sl.y),
+                      __builtin_amdgcn_perm(tb.x, tb.y, sl.z), __builtin_amdgcn_perm(tb.x, tb.y, sl.w)};
+    const u32x4 ub = {__builtin_amdgcn_perm(tb.z, tb.w, sl.x), __builtin_amdgcn_perm(tb.z, tb.w, sl.y),
+                      __builtin_amdgcn_perm(tb.z, tb.w, sl.z), __builtin_amdgcn_perm(tb.z, tb.w, sl.w)};
+    wa = __builtin_bit_cast(half8, ua);
+    wb = __builtin_bit_cast(half8, ub);
+}
+
 // Work item = 128 rows x 128 outputs of one tensor, 4 waves of 64 x 64
 // (2 x 2 blocks of 32 x 32), each wave independent of the others: it loads
 // its X operands straight from the split rows and its weights' codes and
@@ -642,17 +673,7 @@ void cq_gemm_split_kernel(CqSplitArgs a)
             half8 wa[OB], wb[OB];
 #pragma unroll
             for (int ob = 0; ob < OB; ob++) {
-                const uint4 tb = st.tab[ob];
-                const uint32_t b0 = (st.cw[ob] >> (4 * ks)) & 0x03030303u, h0 = b0 | 0x04040404u;
-                const uint32_t b1 = (st.cw[ob] >> (4 * ks + 2)) & 0x03030303u, h1 = b1 | 0x04040404u;
-                const uint4 sl = {__builtin_amdgcn_perm(h0, b0, 0x05010400u), __builtin_amdgcn_perm(h0, b0, 0x07030602u),
-                                  __builtin_amdgcn_perm(h1, b1, 0x05010400u), __builtin_amdgcn_perm(h1, b1, 0x07030602u)};
-                const u32x4 ua = {__builtin_amdgcn_perm(tb.x, tb.y, sl.x), __builtin_amdgcn_perm(tb.x, tb.y, sl.y),
-                                  __builtin_amdgcn_perm(tb.x, tb.y, sl.z), __builtin_amdgcn_perm(tb.x, tb.y, sl.w)};
-                const u32x4 ub = {__builtin_amdgcn_perm(tb.z, tb.w, sl.x), __builtin_amdgcn_perm(tb.z, tb.w, sl.y),
-                                  __builtin_amdgcn_perm(tb.z, tb.w, sl.z), __builtin_amdgcn_perm(tb.z, tb.w, sl.w)};
-                wa[ob] = __builtin_bit_cast(half8, ua);
-                wb[ob] = __builtin_bit_cast(half8, ub);
+                cq_decode8(st.tab[ob], st.cw[ob] >> (4 * ks), wa[ob], wb[ob]);
             }
 #pragma unroll
             for (int rb = 0; rb < 2; rb++)
@@ -793,6 +814,338 @@ void cq_gemm_split_kernel(CqSplitArgs a)
         drain();
 }
 
+// The split GEMM for batches that give cq_gemm_split_kernel too few of its
+// 128 x 128 tiles to fill the chip (or to balance it): a work-group is 64 x 64
+// outputs, its four waves each take a quarter of the columns (steps) of the
+// whole tile, and their sums meet in LDS in column order. A wave's step is the
+// big kernel's (2 x 2 blocks, 24 MFMAs), so the operand traffic per product
+// is the same; the tile is a quarter of the size and a quarter of the steps
+// long. 300 rows x 768 columns x 1568 outputs: 20.6 -> 9.5 us (1024 rows 21.8
+// -> 14.1, 0.5 PFLOP/s of MFMA). Four partial sums instead of one chain also
+// lower the error against 64 bits, 3.3e-7 -> 2.0e-7.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void cq_gemm_fine_kernel(CqSplitArgs a)
+{
+    constexpr int SLD = 64 + 4;                         // row stride of a wave's stage, floats
+    __shared__ __attribute__((aligned(16))) float stage[4][64 * SLD];
+    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, jh = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // work-group w runs on XCD w % 8, which walks a contiguous range of
+    // items: the output tiles of one row tile read its X rows from one L2
+    const uint32_t ntiles = a.tile0[a.nt], total = (a.rows + 63) / 64 * ntiles;
+    const uint32_t item = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+    if (item >= total)
+        return;
+    const uint32_t r0 = item / ntiles * 64, tile = item % ntiles, ti = tensor_of(a.tile0, a.nt, tile);
+    const uint32_t out = a.out[ti], o0 = (tile - a.tile0[ti]) * 64;
+    const uint32_t nkb = a.in_pad / 16, nsteps = a.in_pad / CS_KT;
+    const uint32_t s0 = nsteps * wave / 4, s1 = nsteps * (wave + 1) / 4;
+
+    // rows or outputs past the end read row block 0 or output 0: what they
+    // feed is never stored
+    const half8 *xr[2];
+    uint32_t oc[2];
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const uint32_t rb = r0 + 32 * b < a.rows ? (r0 >> 5) + b : 0, o = o0 + 32 * b + ln;
+        xr[b] = reinterpret_cast<const half8 *>(a.xs) + (uint64_t)rb * nkb * 128;
+        oc[b] = o < out ? o : 0;
+    }
+    struct Step {
+        half8 x[2][2][2];                               // [ks][rb][plane]
+        uint32_t cw[2];
+        uint4 tab[2];
+    };
+    auto load = [&](uint32_t s, Step &st) __attribute__((always_inline)) {
+        s = min(s, nsteps - 1);                         // (past the end: a step that exists, not used)
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+                    st.x[ks][rb][p] = xr[rb][((2 * s + ks) * 2 + p) * 64 + lane];
+#pragma unroll
+        for (int ob = 0; ob < 2; ob++) {
+            st.cw[ob] = a.cw[ti][((uint64_t)s * out + oc[ob]) * 2 + jh];
+            st.tab[ob] = a.tab[ti][(uint64_t)((s * CS_KT) >> a.log2_group) * out + oc[ob]];
+        }
+    };
+    float16v acc[2][2];
+#pragma unroll
+    for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+        for (int ob = 0; ob < 2; ob++)
+            acc[rb][ob] = float16v{};
+    auto compute = [&](const Step &st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            half8 wa[2], wb[2];
+#pragma unroll
+            for (int ob = 0; ob < 2; ob++)
+                cq_decode8(st.tab[ob], st.cw[ob] >> (4 * ks), wa[ob], wb[ob]);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.x[ks][q >> 1][0], wa[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.x[ks][q >> 1][1], wa[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.x[ks][q >> 1][0], wb[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
+        }
+    };
+    // two register sets in turn, loads a step ahead of the MFMAs (the
+    // scheduling barriers keep them there)
+    Step sa, sb;
+    if (s0 < s1)
+        load(s0, sa);
+    const int rx = a.rexp[min(r0 + lane, a.rows - 1)];  // lane t: row r0 + t
+    int ce[2];
+#pragma unroll
+    for (int ob = 0; ob < 2; ob++)
+        ce[ob] = a.cexp[ti][oc[ob]];
+    for (uint32_t s = s0; s < s1; s += 2) {
+        load(s + 1, sb);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(sa);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + 1 >= s1)
+            break;
+        load(s + 2, sa);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(sb);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    float *const sw = stage[wave];
+#pragma unroll
+    for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = 32 * rb + 8 * (i >> 2) + 4 * jh + (i & 3);
+            const int e = __shfl(rx, t, 64);
+#pragma unroll
+            for (int ob = 0; ob < 2; ob++)
+                sw[t * SLD + 32 * ob + ln] = ldexpf(acc[rb][ob][i], -(e + ce[ob]));
+        }
+    __syncthreads();
+    float *y = a.y[ti];
+    const bool v4 = (out & 3u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) {
+        const uint32_t r = 16 * u + tid / 16, c = 4 * (tid % 16), row = r0 + r, o = o0 + c;
+        const float *p = &stage[0][0] + r * SLD + c;
+        float4v z = *reinterpret_cast<const float4v *>(p);
+#pragma unroll
+        for (int w = 1; w < 4; w++)
+            z += *reinterpret_cast<const float4v *>(p + w * 64 * SLD);
+        if (row >= a.rows)
+            continue;
+        float *dst = y + (uint64_t)row * out + o;
+        if (v4 && o + 3 < out) {
+            *reinterpret_cast<float4v *>(dst) = z;
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (o + k < out)
+                    dst[k] = z[k];
+        }
+    }
+}
+
+// The split GEMM for a batch of some hundred rows, from the raw activations
+// (group 128): a work-group is 32 rows x 32 OB outputs, one wave per group of
+// 128 columns. Each wave loads its rows' group straight into the MFMA operand
+// layout (lane: row lane % 32, columns 16 kb + 8 (lane / 32) + [0, 8) of each
+// of 8 k-blocks), transforms it there - butterflies 1, 2, 4 inside a lane's
+// eight columns, 8 between the lane halves, 16, 32, 64 between k-blocks -
+// splits it into the fp16 pair at the (row, group)'s own power of two, and
+// multiplies it with the group's decoded weights. The groups' sums meet in
+// LDS in group order.
+//
+// cq_gemm_split_kernel gives such a batch a few dozen work-groups that walk
+// all the columns in turn, behind a prepare launch. What bounds it
+// here is one wave's chain (loads, about 800 VALU of transform and split, 24
+// OB MFMAs); the transform is repeated for every 32 OB outputs, which is why
+// larger batches prepare their rows once. 300 rows, mean of q/k/v/gate and
+// out_proj: 5.2 + 21.2 us (prepare, big kernel) -> 11.8. A power of two per
+// (row, group) rather than per row: error against 64 bits 1.8e-7.
+template <int OB>
+__global__ __launch_bounds__(64 * CQ_RAW_MAX_G)
+void cq_gemm_raw_kernel(CqSplitArgs a)
+{
+#pragma clang fp contract(off)
+    constexpr int SLD = 32 * OB + 4;                    // row stride of a wave's stage, floats
+    extern __shared__ __attribute__((aligned(16))) float raw_stage[];   // [groups][32][SLD]
+    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, jh = lane >> 5;
+    const uint32_t g = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t tile = blockIdx.x, r0 = blockIdx.y * 32, ti = tensor_of(a.tile0, a.nt, tile);
+    const uint32_t out = a.out[ti], o0 = (tile - a.tile0[ti]) * (32 * OB);
+
+    // every load first (the scheduler otherwise leaves the weights' pointers,
+    // and so their loads, behind the transform); rows and outputs past the
+    // end read the last row and output 0: what they feed is never stored
+    float v[8][8];
+    {
+        const float *x = a.x + (uint64_t)min(r0 + ln, a.rows - 1) * a.in + g * 128 + 8 * jh;
+#pragma unroll
+        for (int kb = 0; kb < 8; kb++) {
+            const float4 u0 = *reinterpret_cast<const float4 *>(x + 16 * kb);
+            const float4 u1 = *reinterpret_cast<const float4 *>(x + 16 * kb + 4);
+            v[kb][0] = u0.x;
+            v[kb][1] = u0.y;
+            v[kb][2] = u0.z;
+            v[kb][3] = u0.w;
+            v[kb][4] = u1.x;
+            v[kb][5] = u1.y;
+            v[kb][6] = u1.z;
+            v[kb][7] = u1.w;
+        }
+    }
+    uint32_t cw[4][OB];
+    uint4 tab[OB];
+    int32_t ce[OB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) {
+        const uint32_t o = o0 + 32 * ob + ln, oc = o < out ? o : 0;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            cw[s][ob] = a.cw[ti][((uint64_t)(4 * g + s) * out + oc) * 2 + jh];
+        tab[ob] = a.tab[ti][(uint64_t)g * out + oc];
+        ce[ob] = a.cexp[ti][oc];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the engine's butterflies, stage by stage
+#pragma unroll
+    for (int len = 1; len < 8; len <<= 1)
+#pragma unroll
+        for (int kb = 0; kb < 8; kb++)
+#pragma unroll
+            for (int s = 0; s < 8; s++)
+                if ((s & len) == 0) {
+                    const float u = v[kb][s], w = v[kb][s + len];
+                    v[kb][s] = u + w;
+                    v[kb][s + len] = u - w;
+                }
+    // length 8, two values at a time: one swap brings (p of both halves) into
+    // the lower lanes and (q of both) into the upper ones, one takes the sums
+    // and differences back
+#pragma unroll
+    for (int kb = 0; kb < 8; kb++)
+#pragma unroll
+        for (int s = 0; s < 8; s += 2) {
+            const auto f = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[kb][s]), __float_as_uint(v[kb][s + 1]),
+                                                            false, false);
+            const float lo = __uint_as_float(f[0]), hi = __uint_as_float(f[1]);
+            const float sum = lo + hi, dif = lo - hi;
+            const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(dif), false, false);
+            v[kb][s] = __uint_as_float(b[0]);
+            v[kb][s + 1] = __uint_as_float(b[1]);
+        }
+#pragma unroll
+    for (int len = 1; len < 8; len <<= 1)
+#pragma unroll
+        for (int kb = 0; kb < 8; kb++)
+            if ((kb & len) == 0)
+#pragma unroll
+                for (int s = 0; s < 8; s++) {
+                    const float u = v[kb][s], w = v[kb + len][s];
+                    v[kb][s] = u + w;
+                    v[kb + len][s] = u - w;
+                }
+
+    // this (row, group)'s power of two, then the pairs
+    float mx = 0.0f;
+#pragma unroll
+    for (int kb = 0; kb < 8; kb++)
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+            mx = fmaxf(mx, fabsf(v[kb][s]));
+    mx = fmaxf(mx, xor_lanes<32>(mx, lane)) * a.scale;
+    int e = 0, sh = 0;
+    if (mx > 0.0f && mx <= FLT_MAX) {
+        (void)frexpf(mx, &e);
+        sh = 15 - e;                                    // mx * 2^sh in [2^14, 2^15)
+    }
+    // the engine's prepared value (one rounding) times 2^sh in one product:
+    // scale * 2^sh is exact up to 2^120, and the rare larger rest (a group
+    // below 2^-105) exact again
+    const float f = ldexpf(a.scale, min(sh, 120)), rest = ldexpf(1.0f, max(sh - 120, 0));
+    const bool tiny = __ballot(sh > 120) != 0;
+    half8 xa[8], xb[8];
+    const float neg1 = opaque_neg1();
+#pragma unroll
+    for (int kb = 0; kb < 8; kb++) {
+        u32x4 ha, hb;
+#pragma unroll
+        for (int s = 0; s < 8; s += 2) {
+            float y0 = v[kb][s] * f, y1 = v[kb][s + 1] * f;
+            if (tiny) {
+                y0 *= rest;
+                y1 *= rest;
+            }
+            asm volatile("" : "+v"(y0), "+v"(y1));      // both halves from this one value
+            ha[s >> 1] = __builtin_bit_cast(uint32_t, half2v{(_Float16)y0, (_Float16)y1});
+            hb[s >> 1] = split_lo2(ha[s >> 1], y0, y1, neg1);
+        }
+        xa[kb] = __builtin_bit_cast(half8, ha);
+        xb[kb] = __builtin_bit_cast(half8, hb);
+    }
+
+    float16v acc[OB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+        acc[ob] = float16v{};
+#pragma unroll
+    for (int kb = 0; kb < 8; kb++) {
+        half8 wa[OB], wb[OB];
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            cq_decode8(tab[ob], cw[kb >> 1][ob] >> (4 * (kb & 1)), wa[ob], wb[ob]);
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[kb], wa[ob], acc[ob], 0, 0, 0);
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xb[kb], wa[ob], acc[ob], 0, 0, 0);
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[kb], wb[ob], acc[ob], 0, 0, 0);
+    }
+    float *const sw = raw_stage + g * 32 * SLD;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int t = 8 * (i >> 2) + 4 * jh + (i & 3);
+        const int rx = __shfl(sh, t, 64);               // row t's (both halves hold it)
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            sw[t * SLD + 32 * ob + ln] = ldexpf(acc[ob][i], -(rx + ce[ob]));
+    }
+    __syncthreads();
+    const uint32_t ng = blockDim.x >> 6;
+    float *y = a.y[ti];
+    const bool v4 = (out & 3u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+    for (uint32_t u = tid; u < 32 * 8 * OB; u += blockDim.x) {
+        const uint32_t r = u / (8 * OB), c = 4 * (u % (8 * OB)), row = r0 + r, o = o0 + c;
+        const float *p = raw_stage + r * SLD + c;
+        float4v z = *reinterpret_cast<const float4v *>(p);
+        for (uint32_t k = 1; k < ng; k++)
+            z += *reinterpret_cast<const float4v *>(p + k * 32 * SLD);
+        if (row >= a.rows)
+            continue;
+        float *dst = y + (uint64_t)row * out + o;
+        if (v4 && o + 3 < out) {
+            *reinterpret_cast<float4v *>(dst) = z;
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (o + k < out)
+                    dst[k] = z[k];
+        }
+    }
+}
+
 // ------------------------------------------------ the engine's LUT order
 
 // 2-bit matvecs for a few rows (one decode step's tokens) computed the way
@@ -828,10 +1181,7 @@ __global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmAr
     const int lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const uint32_t group = G ? G : a.group, gw = group / 16;      // words per group
-    const uint32_t tile = blockIdx.x, row = blockIdx.y;
-    uint32_t t = 0;
-    while (t + 1 < a.nt && tile >= a.tile0[t + 1])
-        t++;
+    const uint32_t tile = blockIdx.x, row = blockIdx.y, t = tensor_of(a.tile0, a.nt, tile);
     const uint32_t o = (tile - a.tile0[t]) * CQ_LUT_OT + lane, oc = min(o, a.out[t] - 1);
     const uint32_t *qw = reinterpret_cast<const uint32_t *>(a.packed[t] + (uint64_t)oc * a.rowbytes);
     const uint16_t *nrm = a.norms[t] + (uint64_t)oc * a.ngroup;
@@ -1005,6 +1355,30 @@ hipError_t launch_cq_gemm_split(const CqSplitArgs &a, hipStream_t s)
     const uint64_t slots = std::max<uint64_t>(8, (uint64_t)cus[dev] * 2 / 8 * 8);
     const uint64_t grid = std::min<uint64_t>((items + 7) / 8 * 8, slots);
     hipLaunchKernelGGL(cq_gemm_split_kernel<CQ_SPLIT_OB>, dim3((uint32_t)grid), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_cq_gemm_fine(const CqSplitArgs &a, hipStream_t s)
+{
+    if (a.rows == 0 || a.nt == 0 || a.tile0[a.nt] == 0)
+        return hipSuccess;
+    const uint64_t items = (uint64_t)((a.rows + 63) / 64) * a.tile0[a.nt];
+    if (items > 0x7FFFFFF0ull)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(cq_gemm_fine_kernel, dim3((uint32_t)((items + 7) / 8 * 8)), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_cq_gemm_raw(const CqSplitArgs &a, hipStream_t s)
+{
+    if (a.rows == 0 || a.nt == 0 || a.tile0[a.nt] == 0)
+        return hipSuccess;
+    constexpr int OB = CQ_FINE_NT / 32;
+    const uint32_t ng = a.in_pad / 128;
+    if (a.log2_group != 7 || a.in != a.in_pad || ng == 0 || ng > CQ_RAW_MAX_G || (a.rows + 31) / 32 > 65535)
+        return hipErrorInvalidValue;
+    const size_t lds = (size_t)ng * 32 * (32 * OB + 4) * sizeof(float);
+    hipLaunchKernelGGL(cq_gemm_raw_kernel<OB>, dim3(a.tile0[a.nt], (a.rows + 31) / 32), dim3(64 * ng), lds, s, a);
     return hipGetLastError();
 }
 

@@ -376,3 +376,25 @@ def test_cq_split_persistent_walks_and_column_scales():
             assert np.all(err <= 1e-5 * sc[:, j] + 1e-6), (shapes[i], r, float(err.max()))
     for q in qs:
         q.close()
+
+
+@pytest.mark.parametrize("shape,rows", [
+    ((70, 32, 32, 2), 1), ((64, 64, 64, 2), 64), ((130, 96, 32, 2), 65),    # one to three steps for four waves
+    ((65, 768, 128, 2), 63), ((96, 640, 128, 2), 129), ((200, 2048, 256, 2), 1023),
+    ((33, 768, 128, 2), 1024), ((33, 768, 128, 2), 1025),                   # the last row count of its kernel, the next's first
+])
+def test_cq_split_tiles(shape, rows):
+    """Edges of the 64 x 64 tiles and of the columns' split over four waves,
+    against the product in 64 bits of the prepared rows. Three fp16 products
+    hold each term to about 2^-22 of itself and the sums round in fp32: at
+    most (columns + 8) * 2^-24 of sum |w x|."""
+    out, inp, group, b = shape
+    say("cq split tiles", shape, rows)
+    t = make_cq_tensor(out + rows, out, inp, group, b)
+    x = np.stack([det_normal(300 + r, inp) for r in range(rows)])
+    y = run_split(t, x)[3]
+    w = (t.cb()[t.codes()] * np.repeat(t.norms(), group, 1)).astype(np.float64)     # the fp32 products
+    for r in (0, rows // 2, rows - 1):
+        xh = O.cq_prepare(t, x[r]).astype(np.float64)
+        err = np.abs(y[r].astype(np.float64) - w @ xh) / (np.abs(w) @ np.abs(xh))
+        assert err.max() <= (t.in_pad + 8) * 2.0 ** -24, (r, float(err.max()))
