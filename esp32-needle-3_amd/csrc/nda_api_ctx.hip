@@ -340,6 +340,31 @@ int hist_reserve(nda_ctx *c, size_t extra)
     return ensure_buf(c, c->d_hist_ops, c->hist_ops_cap, c->hist_pending.size() + extra);
 }
 
+bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &s) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return s != hipStreamCaptureStatusNone;
+}
+
+std::vector<uint32_t> list_key(uint32_t kind, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens,
+                               std::initializer_list<uint32_t> extra)
+{
+    std::vector<uint32_t> k;
+    k.reserve(4 + 2 * (size_t)nseq + extra.size());
+    k.push_back(kind);
+    k.push_back(nseq);
+    k.insert(k.end(), extra);
+    for (uint32_t b = 0; b < nseq; b++)
+        k.push_back(sid(ids, b));
+    if (n_tokens)
+        k.insert(k.end(), n_tokens, n_tokens + nseq);
+    return k;
+}
+
 // Upload seq ids (and optional per-row offsets) for a launch; returns device
 // pointers, null when the identity mapping applies.
 int upload_rows(nda_ctx *c, uint32_t rows, const uint32_t *row_seq, const uint32_t *row_t,
@@ -352,6 +377,7 @@ int upload_rows(nda_ctx *c, uint32_t rows, const uint32_t *row_seq, const uint32
     int rc = ensure_rows(c, rows);
     if (rc)
         return rc;
+    c->rows_list.what.clear();
     if (row_seq) {
         if (int rc2 = upload(c, c->d_rows, row_seq, rows * sizeof(uint32_t), st))
             return rc2;

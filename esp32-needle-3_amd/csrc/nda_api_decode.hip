@@ -283,23 +283,30 @@ static int prefix_pass(nda_ctx *c, const AttnArgs &a, uint32_t nseq, const uint3
 {
     const uint64_t trows = 32u * PREFIX_PASS_WAVES;
     const uint32_t per_head = (uint32_t)(((uint64_t)nseq * c->geo.rep + trows - 1) / trows);
-    std::vector<uint32_t> items;
-    items.reserve(8 * (size_t)ps.n_items);
     const uint32_t seq0 = sid(ids, 0);
-    for (uint32_t g = 0; g < c->cfg.n_kv_heads; g++)
-        for (uint32_t t = 0; t < per_head; t++) {
-            // sequence, kv-head, row tile, first row, rows, position (unused),
-            // prefix slots, prefix id; the sequence only names a page-table
-            // row, which a pass with no own tiles never reads
-            const uint32_t rec[8] = {seq0, g, t, 0u, nseq, ps.n_sh, ps.n_sh, (uint32_t)ps.prefix};
-            items.insert(items.end(), rec, rec + 8);
+    // the list a step's first layer uploaded serves the others (it is made
+    // of these values alone)
+    const std::vector<uint32_t> key = {LIST_PREFIX_PASS, seq0, nseq, ps.n_sh, (uint32_t)ps.prefix};
+    if (!c->pf_list.holds(key, c->pf_cap, st)) {
+        std::vector<uint32_t> items;
+        items.reserve(8 * (size_t)ps.n_items);
+        for (uint32_t g = 0; g < c->cfg.n_kv_heads; g++)
+            for (uint32_t t = 0; t < per_head; t++) {
+                // sequence, kv-head, row tile, first row, rows, position (unused),
+                // prefix slots, prefix id; the sequence only names a page-table
+                // row, which a pass with no own tiles never reads
+                const uint32_t rec[8] = {seq0, g, t, 0u, nseq, ps.n_sh, ps.n_sh, (uint32_t)ps.prefix};
+                items.insert(items.end(), rec, rec + 8);
+            }
+        while ((items.size() / 8) % 8) {
+            const uint32_t pad[8] = {0xFFFFFFFFu, 0, 0, 0, 0, 0, 0, 0};
+            items.insert(items.end(), pad, pad + 8);
         }
-    while ((items.size() / 8) % 8) {
-        const uint32_t pad[8] = {0xFFFFFFFFu, 0, 0, 0, 0, 0, 0, 0};
-        items.insert(items.end(), pad, pad + 8);
+        c->pf_list.what.clear();
+        if (int rc = upload(c, c->d_pf, items.data(), items.size() * 4, st))
+            return rc;
+        c->pf_list.set(key, c->pf_cap, st);
     }
-    if (int rc = upload(c, c->d_pf, items.data(), items.size() * 4, st))
-        return rc;
     PrefillArgs pa{};
     pa.q = a.q;
     pa.pool = a.pool;
@@ -312,7 +319,7 @@ static int prefix_pass(nda_ctx *c, const AttnArgs &a, uint32_t nseq, const uint3
     pa.part_stride = c->cfg.v_head_dim + 2;
     pa.tab_cap = (ps.n_sh + 31) / 32;         // the prefix's tiles only
     pa.pg = a.pg;
-    pa.n_items = (uint32_t)(items.size() / 8);
+    pa.n_items = ps.n_items;
     pa.nh = a.nh;
     pa.qscale = a.qscale;
     ProfScope ps_(c, NDA_K_DECODE, st);

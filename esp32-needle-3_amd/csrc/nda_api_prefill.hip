@@ -92,6 +92,11 @@ static uint32_t prefill_ksplit(const nda_ctx *c, size_t items, uint32_t tiles, i
 
 int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens, PrefillPlan &pl)
 {
+    std::vector<uint32_t> key = list_key(LIST_ITEMS, nseq, ids, n_tokens);
+    if (c->plan_ver == c->state_ver && c->plan_key == key) {
+        pl = c->plan;
+        return NDA_OK;
+    }
     pl = PrefillPlan();
     pl.nseq = nseq;
     for (uint32_t b = 0; b < nseq; b++) {
@@ -132,6 +137,9 @@ int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t 
     pl.n_items = 8 * (size_t)prefill_bins(c, nseq, ids, n_tokens, pl.rep, pl.trows, bins, &items);
     if (!pl.valu)
         pl.ksplit = prefill_ksplit(c, items, pl.tab_cap, pl.waves);
+    c->plan = pl;
+    c->plan_key = std::move(key);
+    c->plan_ver = c->state_ver;
     return NDA_OK;
 }
 
@@ -201,17 +209,21 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
         if (n_tokens[b])
             s.stored_end = std::max(s.stored_end, s.pos + n_tokens[b]);
     }
-    std::vector<uint32_t> rseq(rows), rt(rows);
-    for (uint32_t b = 0, r = 0; b < nseq; b++)
-        for (uint32_t t = 0; t < n_tokens[b]; t++, r++) {
-            rseq[r] = sid(ids, b);
-            rt[r] = t;
-        }
     if (int rc = sync_tables(c, st))
         return rc;
-    const uint32_t *d_seq, *d_t;
-    if (int rc = upload_rows(c, (uint32_t)rows, rseq.data(), rt.data(), st, &d_seq, &d_t))
-        return rc;
+    const uint32_t *d_seq = c->d_rows, *d_t = c->d_rows + rows;
+    const std::vector<uint32_t> rows_key = list_key(LIST_ROWS, nseq, ids, n_tokens);
+    if (!c->rows_list.holds(rows_key, c->rows_cap, st)) {
+        std::vector<uint32_t> rseq(rows), rt(rows);
+        for (uint32_t b = 0, r = 0; b < nseq; b++)
+            for (uint32_t t = 0; t < n_tokens[b]; t++, r++) {
+                rseq[r] = sid(ids, b);
+                rt[r] = t;
+            }
+        if (int rc = upload_rows(c, (uint32_t)rows, rseq.data(), rt.data(), st, &d_seq, &d_t))
+            return rc;
+        c->rows_list.set(rows_key, c->rows_cap, st);
+    }
     {
         AppendArgs a{};
         a.k = k;
@@ -240,32 +252,39 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
     // position, shared-prefix slots, prefix id (-1: none).
     // in the order of prefill_bins (the same as planned: positions have not
     // changed since)
-    std::vector<uint32_t> tok0(nseq);
-    for (uint32_t b = 0, tok = 0; b < nseq; b++) {
-        tok0[b] = tok;
-        tok += n_tokens[b];
-    }
-    std::vector<std::array<uint32_t, 3>> bins[8];
-    const uint32_t per_bin = prefill_bins(c, nseq, ids, n_tokens, rep, trows, bins);
-    std::vector<uint32_t> items;
-    items.reserve(8 * 8 * (size_t)per_bin);
-    for (const auto &bin : bins) {
-        for (const auto &it : bin) {
-            const uint32_t b = it[0], qq = sid(ids, b);
-            const SeqHost &s = c->seqs[qq];
-            const Vis v = visible(s, s.pos, c->cfg.window);
-            const uint32_t rec[8] = {qq, it[1], it[2], tok0[b], n_tokens[b], s.pos, v.n_sh, (uint32_t)s.prefix};
-            items.insert(items.end(), rec, rec + 8);
+    // Of the plan alone, so a step's other layers take the list as it is.
+    const std::vector<uint32_t> key = list_key(LIST_ITEMS, nseq, ids, n_tokens,
+                                               {(uint32_t)c->state_ver, (uint32_t)(c->state_ver >> 32)});
+    if (!c->pf_list.holds(key, c->pf_cap, st)) {
+        std::vector<uint32_t> tok0(nseq);
+        for (uint32_t b = 0, tok = 0; b < nseq; b++) {
+            tok0[b] = tok;
+            tok += n_tokens[b];
         }
-        for (size_t n = bin.size(); n < per_bin; n++) {
-            const uint32_t pad[8] = {0xFFFFFFFFu, 0, 0, 0, 0, 0, 0, 0};
-            items.insert(items.end(), pad, pad + 8);
+        std::vector<std::array<uint32_t, 3>> bins[8];
+        const uint32_t per_bin = prefill_bins(c, nseq, ids, n_tokens, rep, trows, bins);
+        std::vector<uint32_t> items;
+        items.reserve(8 * 8 * (size_t)per_bin);
+        for (const auto &bin : bins) {
+            for (const auto &it : bin) {
+                const uint32_t b = it[0], qq = sid(ids, b);
+                const SeqHost &s = c->seqs[qq];
+                const Vis v = visible(s, s.pos, c->cfg.window);
+                const uint32_t rec[8] = {qq, it[1], it[2], tok0[b], n_tokens[b], s.pos, v.n_sh, (uint32_t)s.prefix};
+                items.insert(items.end(), rec, rec + 8);
+            }
+            for (size_t n = bin.size(); n < per_bin; n++) {
+                const uint32_t pad[8] = {0xFFFFFFFFu, 0, 0, 0, 0, 0, 0, 0};
+                items.insert(items.end(), pad, pad + 8);
+            }
         }
+        if (items.size() != 8 * pl.n_items)
+            return fail(c, NDA_ERR_STATE, "prefill work list: size differs from its plan");
+        c->pf_list.what.clear();
+        if (int rc = upload(c, c->d_pf, items.data(), items.size() * 4, st))
+            return rc;
+        c->pf_list.set(key, c->pf_cap, st);
     }
-    if (items.size() != 8 * pl.n_items)
-        return fail(c, NDA_ERR_STATE, "prefill work list: size differs from its plan");
-    if (int rc = upload(c, c->d_pf, items.data(), items.size() * 4, st))
-        return rc;
     PrefillArgs pa{};
     pa.q = q;
     pa.gate = gate;
@@ -283,7 +302,7 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
         pa.part_stride = PF_PART_STRIDE;
     }
     pa.pg = c->pg;
-    pa.n_items = (uint32_t)(items.size() / 8);
+    pa.n_items = (uint32_t)pl.n_items;
     pa.nh = c->cfg.n_heads;
     pa.qscale = (float)(1.4426950408889634 / std::sqrt((double)c->cfg.qk_head_dim));
     ProfScope ps(c, NDA_K_PREFILL, st);

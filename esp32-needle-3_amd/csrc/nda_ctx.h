@@ -43,6 +43,41 @@ struct UploadRec {
     hipEvent_t ev;
 };
 
+// What one nda_prefill call launches: rows, the visible runs they attend,
+// the kernel (VALU or MFMA) and the MFMA work-group size and work list.
+struct PrefillPlan {
+    uint64_t rows = 0, sum_total = 0;
+    uint32_t max_total = 0, rep = 1, trows = 0, nseq = 0;
+    int waves = 4;
+    bool valu = false;
+    size_t n_items = 0;
+    uint32_t tab_cap = 0;               // key tiles of the longest item
+    uint32_t ksplit = 0;                // parts per item's key tiles (0: whole)
+};
+
+// A list in a device buffer that several calls use: `what` it was built from
+// (its kind first, then the values), and the buffer's capacity, which grows
+// whenever the buffer is replaced. Empty: the buffer holds something else. A
+// stream being captured neither takes a list as held nor leaves one: the
+// graph's replays bring their own.
+bool capturing(hipStream_t st);
+struct DevList {
+    std::vector<uint32_t> what;
+    size_t cap = 0;
+    bool holds(const std::vector<uint32_t> &w, size_t c, hipStream_t st) const
+    {
+        return cap == c && what == w && !capturing(st);
+    }
+    void set(const std::vector<uint32_t> &w, size_t c, hipStream_t st)
+    {
+        what.clear();
+        if (!capturing(st)) {
+            what = w;
+            cap = c;
+        }
+    }
+};
+
 constexpr size_t UPLOAD_RING_BYTES = 16u << 20;
 constexpr int UPLOAD_EVENTS = 256;
 
@@ -62,12 +97,19 @@ struct nda_ctx {
     SeqDev *d_seqs = nullptr;
     uint32_t *d_rows = nullptr;         // row_seq | row_t staging
     size_t rows_cap = 0;
+    DevList rows_list;                  // what d_rows holds, where a prefill wrote it
     float *d_part = nullptr;
     size_t part_cap = 0;                // floats
     uint8_t *d_stage = nullptr;
     size_t stage_cap = 0;
     uint32_t *d_pf = nullptr;           // prefill work list staging
     size_t pf_cap = 0;                  // uint32 entries
+    DevList pf_list;                    // the work list that d_pf holds
+    // the last planned prefill: its sequences and token counts, the state
+    // version it was planned at, and the plan before prefill_reserve
+    std::vector<uint32_t> plan_key;
+    uint64_t plan_ver = 0;
+    nda_host::PrefillPlan plan;
     float *d_pf_part = nullptr;         // states of a split-key prefill
     size_t pf_part_cap = 0;             // floats
     // GQA decode work order (longest rows first) for batches of sequences
@@ -99,6 +141,7 @@ struct nda_ctx {
     size_t qfront_cap = 0;              // floats
     uint32_t *d_front_rows = nullptr;   // row_seq | row_t | row_n
     size_t front_rows_cap = 0;          // uint32 entries
+    DevList front_list;                 // what d_front_rows holds
     HistOp *d_hist_ops = nullptr;
     size_t hist_ops_cap = 0;
     std::vector<HistOp> hist_pending;   // applied in order before the next front launch
@@ -283,17 +326,14 @@ int decode_impl(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
                 const float *k, const float *v, const float *gate, float *out, void *stream);
 
 // prefill (nda_api_prefill.hip)
-// What one nda_prefill call launches: rows, the visible runs they attend,
-// the kernel (VALU or MFMA) and the MFMA work-group size and work list.
-struct PrefillPlan {
-    uint64_t rows = 0, sum_total = 0;
-    uint32_t max_total = 0, rep = 1, trows = 0, nseq = 0;
-    int waves = 4;
-    bool valu = false;
-    size_t n_items = 0;
-    uint32_t tab_cap = 0;               // key tiles of the longest item
-    uint32_t ksplit = 0;                // parts per item's key tiles (0: whole)
-};
+// The calls of a step's layers launch the same batch one after another; what
+// they share (the plan, the row list, the work list) is made and uploaded
+// once, told apart by value: the listed sequences, their token counts and the
+// state version. A kind per list, its first value.
+enum : uint32_t { LIST_ROWS = 1, LIST_FRONT, LIST_ITEMS, LIST_PREFIX_PASS };
+// {kind, nseq, extra values, sequences, token counts (none: 1 each)}
+std::vector<uint32_t> list_key(uint32_t kind, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens,
+                               std::initializer_list<uint32_t> extra = {});
 constexpr uint32_t PF_MAX_PARTS = 64;
 constexpr uint32_t PF_PART_STRIDE = 68; // a split part's floats: 64 sums, max, weight sum, padded to 16 bytes
 int prefill_check(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t *n_tokens);
