@@ -53,7 +53,8 @@ static const uint32_t *decode_order(nda_ctx *c, uint32_t rows, hipStream_t st)
 // profiling events (nda_decode_noalloc records none: creating an event may
 // allocate). ordered: the GQA decode may take the rows longest first (it then
 // builds or reuses the context's order buffer; nda_decode_noalloc does not).
-int run_attend(nda_ctx *c, AttnArgs &a, hipStream_t st, float *part, bool prof, bool ordered)
+int run_attend(nda_ctx *c, AttnArgs &a, hipStream_t st, float *part, bool prof, bool ordered,
+               const FrontArgs *front)
 {
     if (mfma_decode(c, a)) {
         PrefillArgs pa{};
@@ -75,7 +76,7 @@ int run_attend(nda_ctx *c, AttnArgs &a, hipStream_t st, float *part, bool prof, 
         if (ordered && !a.row_seq && pa.n_items >= 4u * (uint32_t)c->cus)
             pa.items = decode_order(c, a.rows, st);
         ProfScope ps(c, NDA_K_DECODE, st, prof);
-        hipError_t e = launch_decode_mfma(c->geo, pa, mfma_decode_waves(c, a.rows), st);
+        hipError_t e = launch_decode_mfma(c->geo, pa, mfma_decode_waves(c, a.rows), front, st);
         if (e != hipSuccess)
             return hip_fail(c, e, "decode (MFMA) kernel launch");
         return NDA_OK;
@@ -161,13 +162,8 @@ int nda_kv_append(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids
 
 namespace nda_host {
 
-// Decode, optionally with the append of this position fused in (k/v set).
-// What nda_decode and nda_decode_noalloc check before any launch: arguments,
-// and every visible slot backed (written by an append, a write or an attach;
-// an unbacked one means the caller skipped the append). Returns the longest
-// visible run and the sum over the listed sequences.
-static int decode_check(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, const float *q,
-                        float *out, uint32_t *max_total, uint64_t *sum_total)
+int decode_check(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, const float *q,
+                 float *out, uint32_t *max_total, uint64_t *sum_total)
 {
     if (!c || (nseq && (!q || !out)))
         return c ? fail(c, NDA_ERR_ARG, "null q/out") : NDA_ERR_ARG;
@@ -362,6 +358,7 @@ static int decode_reserve(nda_ctx *c, uint32_t nseq, const uint32_t *ids, uint32
     return NDA_OK;
 }
 
+// Decode, optionally with the append of this position fused in (k/v set).
 int decode_impl(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, const float *q,
                        const float *k, const float *v, const float *gate, float *out, void *stream)
 {

@@ -311,6 +311,14 @@ int nda_attention(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids
     a.hist_write = 1;
     a.pool = c->pool + (uint64_t)layer * c->pg.layer_bytes;
     a.page_table = c->d_pages;
+    AttnArgs d = attn_args(c, layer, nseq, c->d_qfront, gate, out, max_total, sum_total);
+    d.row_seq = d_seq;
+    if (mfma_decode(c, d) && mfma_decode_waves(c, nseq) > 1) {
+        // a GQA batch of few rows: the decode runs the front itself
+        if (int rc = decode_check(c, layer, nseq, ids, d.q, out, &max_total, &sum_total))
+            return rc;
+        return run_attend(c, d, st, nullptr, true, true, &a);
+    }
     {
         ProfScope ps(c, NDA_K_FRONT, st);
         hipError_t e = launch_front(c->geo, a, st);

@@ -315,8 +315,16 @@ int reserve_attend(nda_ctx *c, uint32_t rows, bool staged, uint32_t max_total, u
 // profiling events (nda_decode_noalloc records none: creating an event may
 // allocate). ordered: the GQA decode may take the rows longest first (it then
 // builds or reuses the context's order buffer; nda_decode_noalloc does not).
+// front: the rows' attention front, run by the decode launch itself (only
+// where mfma_decode takes several waves).
 int run_attend(nda_ctx *c, AttnArgs &a, hipStream_t st, float *part = nullptr, bool prof = true,
-               bool ordered = true);
+               bool ordered = true, const FrontArgs *front = nullptr);
+// What nda_decode and nda_decode_noalloc check before any launch: arguments,
+// and every visible slot backed (written by an append, a write or an attach;
+// an unbacked one means the caller skipped the append). Returns the longest
+// visible run and the sum over the listed sequences.
+int decode_check(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, const float *q,
+                 float *out, uint32_t *max_total, uint64_t *sum_total);
 
 // ---- shared between the ABI groups
 

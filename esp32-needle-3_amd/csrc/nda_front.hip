@@ -27,182 +27,32 @@
 // Every multiply and add rounds on its own (no contraction) and divide / sqrt
 // are correctly rounded, so the results are bit-identical to the engine's
 // host build, and so are the int8 codes computed from them.
-#include "nda_device.h"
+#include "nda_front.h"
 
 #include <algorithm>
 
 namespace nda {
 
-template <int DK, int DV, int REP>
-struct FrontShape {
-    static constexpr int NC = REP * DK + DK + DV;   // columns of one kv group
-    static constexpr int NG = NC / 4;               // four-column groups, one per thread
-    static constexpr int W = (NG + 63) / 64;        // waves per work-group
-    static constexpr int NH = REP + 1;              // normalised heads: REP q + 1 k
-    static constexpr int STRIDE = DK + 4;           // LDS row: 16-byte aligned, banks spread
-    static constexpr int HALF = DK / 2;
-    static constexpr int TREG = 4;                  // taps held in registers; more are streamed
-    static_assert(DK % 4 == 0 && DV % 4 == 0, "four-column groups");
-    static_assert(W <= 4, "one group per thread");
-};
-
-typedef float float4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
-
-__device__ __forceinline__ void acc4(float4 &a, const float4 &w, const float4 &x)
-{
-#pragma clang fp contract(off)
-    a.x = a.x + w.x * x.x;
-    a.y = a.y + w.y * x.y;
-    a.z = a.z + w.z * x.z;
-    a.w = a.w + w.w * x.w;
-}
-
 template <int ES, int DK, int DV, int REP>
 __global__ __launch_bounds__((64 * FrontShape<DK, DV, REP>::W)) void front_kernel(FrontArgs a)
 {
-#pragma clang fp contract(off)
     using S = FrontShape<DK, DV, REP>;
-    __shared__ __align__(16) float ylds[S::NH * S::STRIDE];   // conv outputs of the q/k heads
-    __shared__ __align__(16) float sqlds[S::NH * S::STRIDE];  // their squares
-    __shared__ __align__(16) float vlds[DV];
-    __shared__ float invlds[S::NH];
+    __shared__ FrontLds<DK, DV, REP> lds;
 
-    const uint32_t nkv = a.nkv;
-    const uint32_t row = blockIdx.x / nkv, g = blockIdx.x % nkv;
+    const uint32_t row = blockIdx.x / a.nkv, g = blockIdx.x % a.nkv;
     const int tid = threadIdx.x;
     const uint32_t seq = a.row_seq ? a.row_seq[row] : row;
     const uint32_t t = a.row_t ? a.row_t[row] : 0u;
     const SeqDev sd = a.seqs[seq];
     const uint32_t pos = (uint32_t)sd.pos + t;
-    const uint32_t taps = a.taps;
-    const uint32_t nt = min(taps, pos + 1u);
-    const uint32_t dq = nkv * REP * DK, dk = nkv * DK, dv = nkv * DV, dcol = dq + dk + dv;
-    float *hist = a.hist + ((uint64_t)seq * a.n_layers + a.layer) * taps * dcol;
     const bool store = a.k_out == nullptr;
-
-    // What steps 3 and 4 read (this thread's rotary pairs and norm scales,
-    // the page of the stored slot) is requested now, beside the tap loads,
-    // so the wave waits on one round of loads rather than three.
-    constexpr int NE = (S::NH * S::HALF + 64 * S::W - 1) / (64 * S::W);   // emit elements per thread
-    const float2 *rope = a.rope + (uint64_t)pos * S::HALF;
-    float2 cs_e[NE];
-    float s1_e[NE], s2_e[NE];
-#pragma unroll
-    for (int n = 0; n < NE; n++) {
-        const int e = tid + n * 64 * S::W;
-        const int h = e / S::HALF, i = e % S::HALF;
-        if (e < S::NH * S::HALF) {
-            const float *sn = a.norm + (h < REP ? 0 : DK);
-            cs_e[n] = rope[i];
-            s1_e[n] = sn[i];
-            s2_e[n] = sn[i + S::HALF];
-        }
-    }
     int slot = 0;
-    int32_t page = -1;
+    int32_t page = -1;      // of the stored slot, requested beside the front's loads
     if (store) {
         slot = own_slot(sd, (int)pos, (int)a.pg.window);
         page = a.page_table[(uint64_t)seq * a.pg.pages_per_seq + (slot >> a.pg.log2_page)];
     }
-
-    // 1. tap convolution of this thread's four columns
-    const bool active = tid < S::NG;
-    const int lc = tid * 4;                      // column within the group
-    const float *src;
-    uint32_t ld, cc, gc;                         // source row length, column in it, column in dcol
-    if (lc < REP * DK) {
-        src = a.q; ld = dq; cc = g * REP * DK + lc; gc = cc;
-    } else if (lc < REP * DK + DK) {
-        src = a.k; ld = dk; cc = g * DK + (lc - REP * DK); gc = dq + cc;
-    } else {
-        src = a.v; ld = dv; cc = g * DV + (lc - REP * DK - DK); gc = dq + dk + cc;
-    }
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float4 raw = acc;
-    if (active) {
-        float4 x[S::TREG], w[S::TREG];
-        raw = ld4(src + (uint64_t)row * ld + cc);
-#pragma unroll
-        for (int j = 0; j < S::TREG; j++) {
-            if ((uint32_t)j < nt) {
-                w[j] = ld4(a.w + (uint64_t)j * dcol + gc);
-                if (j == 0)
-                    x[j] = raw;
-                else if ((uint32_t)j <= t)
-                    x[j] = ld4(src + (uint64_t)(row - j) * ld + cc);
-                else
-                    x[j] = ld4(hist + (uint64_t)((pos - j) % taps) * dcol + gc);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < S::TREG; j++)
-            if ((uint32_t)j < nt)
-                acc4(acc, w[j], x[j]);
-        for (uint32_t j = S::TREG; j < nt; j++) {
-            const float4 wj = ld4(a.w + (uint64_t)j * dcol + gc);
-            const float4 xj = j <= t ? ld4(src + (uint64_t)(row - j) * ld + cc)
-                                     : ld4(hist + (uint64_t)((pos - j) % taps) * dcol + gc);
-            acc4(acc, wj, xj);
-        }
-        // the raw row into the tap history, read again only at the next
-        // step's front: streamed past L2 (2-6% off the 4096-row front)
-        if (a.hist_write)
-            __builtin_nontemporal_store(float4v{raw.x, raw.y, raw.z, raw.w},
-                                        reinterpret_cast<float4v *>(hist + (uint64_t)(pos % taps) * dcol + gc));
-        if (lc < (REP + 1) * DK) {
-            const int o = (lc / DK) * S::STRIDE + lc % DK;
-            *reinterpret_cast<float4 *>(ylds + o) = acc;
-            *reinterpret_cast<float4 *>(sqlds + o) =
-                make_float4(acc.x * acc.x, acc.y * acc.y, acc.z * acc.z, acc.w * acc.w);
-        } else if (store) {
-            *reinterpret_cast<float4 *>(vlds + (lc - (REP + 1) * DK)) = acc;
-        } else {
-            *reinterpret_cast<float4 *>(a.v_out + (uint64_t)row * dv + cc) = acc;
-        }
-    }
-    __syncthreads();
-
-    // 2. per-head sum of squares in index order, inverse RMS
-    if (tid < S::NH) {
-        const float *r = sqlds + tid * S::STRIDE;
-        float ss = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DK; i++)
-            ss = ss + r[i];
-        invlds[tid] = 1.0f / __builtin_sqrtf(ss / (float)DK + 1e-6f);
-    }
-    __syncthreads();
-
-    // 3. (1 + s) * x * inv, rotated by the position's (cos, sin)
-#pragma unroll
-    for (int n = 0; n < NE; n++) {
-        const int e = tid + n * 64 * S::W;
-        if (e >= S::NH * S::HALF)
-            break;
-        const int h = e / S::HALF, i = e % S::HALF;
-        const bool is_q = h < REP;
-        float *r = ylds + h * S::STRIDE;
-        const float iv = invlds[h];
-        const float x1 = (1.0f + s1_e[n]) * r[i] * iv;
-        const float x2 = (1.0f + s2_e[n]) * r[i + S::HALF] * iv;
-        const float2 cs = cs_e[n];
-        const float o1 = x1 * cs.x - x2 * cs.y;
-        const float o2 = x2 * cs.x + x1 * cs.y;
-        if (is_q) {
-            float *qo = a.q_out + (uint64_t)row * dq + (g * REP + h) * DK;
-            qo[i] = o1;
-            qo[i + S::HALF] = o2;
-        } else if (store) {
-            r[i] = o1;
-            r[i + S::HALF] = o2;
-        } else {
-            float *ko = a.k_out + (uint64_t)row * dk + g * DK;
-            ko[i] = o1;
-            ko[i + S::HALF] = o2;
-        }
-    }
+    front_steps<DK, DV, REP, 64 * S::W, false>(a, row, g, seq, t, pos, tid, lds);
     if (!store)
         return;
     __syncthreads();
@@ -214,8 +64,8 @@ __global__ __launch_bounds__((64 * FrontShape<DK, DV, REP>::W)) void front_kerne
     if (page < 0)
         return;   // the host backs every stored slot; never taken
     uint8_t *hb = a.pool + (uint64_t)page * a.pg.page_bytes + (uint64_t)g * a.pg.head_bytes;
-    const float kx = tid < DK ? ylds[REP * S::STRIDE + tid] : 0.0f;
-    const float vx = tid < DV ? vlds[tid] : 0.0f;
+    const float kx = tid < DK ? lds.y[REP * S::STRIDE + tid] : 0.0f;
+    const float vx = tid < DV ? lds.v[tid] : 0.0f;
     store_row<ES>(hb, slot & (P - 1), P, kx, vx, tid, DK, DV);
 }
 

@@ -298,9 +298,10 @@ uint32_t pf_tab_max_bytes(int waves, bool dma);
 hipError_t launch_pf_merge(const PrefillArgs &a, uint64_t units, hipStream_t s);
 /* GQA decode on MFMA: `waves` waves (1, 4 or 8) per (row, kv-head) item,
  * n_items = rows * nkv, items in (row, kv-head) order; a.row_seq as in
- * AttnArgs. */
+ * AttnArgs. f (4 or 8 waves; its rows are a's): run the attention front of
+ * the rows first and store their k and v; a.q and f's outputs are not used. */
 bool decode_mfma_supported(const Geo &g);
-hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, int waves, hipStream_t s);
+hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, int waves, const FrontArgs *f, hipStream_t s);
 hipError_t launch_combine(const Geo &g, const AttnArgs &a, hipStream_t s);
 hipError_t launch_copy(const Geo &g, const CopyArgs &a, hipStream_t s);
 hipError_t launch_gather(const Geo &g, const StageArgs &a, hipStream_t s);

@@ -25,7 +25,7 @@
 // per-(slot, kv-head) scales applied to S (k scale) and folded into P (v
 // scale), the engine's dequantisation (engine/src/nd_model.c:2179-2180,
 // :2250-2252).
-#include "nda_device.h"
+#include "nda_front.h"
 
 #include <algorithm>
 #include <float.h>
@@ -1095,15 +1095,20 @@ __device__ __forceinline__ float4v mfma16k32(half8 a, half8 b, float4v c)
 // with eight; one session 23.9 us on the VALU kernel, 5.2 here), so its
 // work-groups split a row's tiles over NW waves, each with its own buffer and
 // softmax state, which meet in LDS at the end. Such a launch may also store
-// the new row first (a.k_new, as the VALU kernel's fused append).
+// the new row first (a.k_new, as the VALU kernel's fused append), or run the
+// row's attention front (FRONT: f's raw projections; q stays in LDS): the
+// front's own launch of two-wave work-groups costs about 4 us, most of it
+// start-up and its loads' latency, which here passes beside the first tile's.
 //
 // RUN (pages of 16 slots, K + V + scales of a kv-head within 128 chunks of
 // 16 bytes): a half tile is a whole kv-head block of one page, 1920 bytes at
 // qk 48, read as one contiguous run by two loads.
-template <int DK, int DV, int REP, bool RUN, int NW>
+struct NoFront {};
+template <int DK, int DV, int REP, bool RUN, int NW, bool FRONT = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW >= 8 ? 2 : 4)))
-void decode_mfma_kernel(PrefillArgs a)
+void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFront> f)
 {
+    static_assert(!FRONT || NW > 1, "the front runs in the several-wave variants");
     static_assert(DK % 16 == 0 && DK <= 64 && DV == 64 && REP <= 16,
                   "decode tiles: dk multiple of 16 up to 64, dv 64, rep <= 16");
     static_assert(!RUN || DK + DV + 8 <= 128, "a kv-head block of a 16-slot page within two loads");
@@ -1281,7 +1286,28 @@ void decode_mfma_kernel(PrefillArgs a)
     TileRef tref;
     Stage sg;
     fetch(tile0, tref);
-    load(tref, sg);
+    // (the tile that holds the row's own slot only after the store)
+    const int slot = FRONT ? own_slot(sd, sd.pos, (int)a.pg.window) : 0;
+    const bool early = !FRONT || tile0 != tiles_sh + slot / PF_KT;
+    if (early)
+        load(tref, sg);
+    const float *qlds = nullptr;
+    if constexpr (FRONT) {
+        using S = FrontShape<DK, DV, REP>;
+        __shared__ FrontLds<DK, DV, REP> fl;
+        const int32_t page = own[slot >> a.pg.log2_page];
+        front_steps<DK, DV, REP, 64 * NW, true>(f, b, kvh, seq, 0u, (uint32_t)sd.pos, threadIdx.x, fl);
+        __syncthreads();
+        if (wave == 0 && page >= 0) {
+            uint8_t *hb = const_cast<uint8_t *>(a.pool) + (uint64_t)page * a.pg.page_bytes + (uint64_t)kvh * a.pg.head_bytes;
+            const float kx = lane < DK ? fl.y[REP * S::STRIDE + lane] : 0.0f, vx = lane < DV ? fl.v[lane] : 0.0f;
+            store_row<1>(hb, slot & (P - 1), P, kx, vx, lane, DK, DV);
+        }
+        __syncthreads();
+        qlds = fl.y + min(r, REP - 1) * S::STRIDE;
+        if (!early)
+            load(tref, sg);
+    }
     fetch(tile0 + 1, tref);
 
     // Q^T operand, hi and lo: column r, dims 32 s + 8 g + [0, 8) and the tail
@@ -1293,7 +1319,7 @@ void decode_mfma_kernel(PrefillArgs a)
     half8 qh[NS + TAIL], ql[NS + TAIL], qx[EXACT ? NS + TAIL : 1];
     int qexp = 0;
     {
-        const float *qr = a.q + qrow * DK;
+        const float *qr = FRONT ? qlds : a.q + qrow * DK;
         const float qs = rvalid ? a.qscale : 0.0f;
         float x[NS + TAIL][8];
 #pragma unroll
@@ -1663,29 +1689,34 @@ bool decode_mfma_supported(const Geo &g)
 }
 
 template <int DK, int DV, int REP, bool RUN>
-static void launch_dec(const PrefillArgs &a, int waves, hipStream_t s)
+static void launch_dec(const PrefillArgs &a, int waves, const FrontArgs *f, hipStream_t s)
 {
-    if (waves == 8)
-        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 8>), dim3(a.n_items), dim3(512), 0, s, a);
+    const dim3 grid(a.n_items);
+    if (waves == 8 && f)
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 8, true>), grid, dim3(512), 0, s, a, *f);
+    else if (waves == 8)
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 8>), grid, dim3(512), 0, s, a, NoFront());
+    else if (waves == 4 && f)
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 4, true>), grid, dim3(256), 0, s, a, *f);
     else if (waves == 4)
-        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 4>), dim3(a.n_items), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 4>), grid, dim3(256), 0, s, a, NoFront());
     else
-        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 1>), dim3(a.n_items), dim3(64), 0, s, a);
+        hipLaunchKernelGGL((decode_mfma_kernel<DK, DV, REP, RUN, 1>), grid, dim3(64), 0, s, a, NoFront());
 }
 
-hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, int waves, hipStream_t s)
+hipError_t launch_decode_mfma(const Geo &g, const PrefillArgs &a, int waves, const FrontArgs *f, hipStream_t s)
 {
     if (a.n_items == 0)
         return hipSuccess;
-    if (a.k_new && waves == 1)
+    if ((a.k_new || f) && waves == 1)
         return hipErrorInvalidValue;        // only the several-wave variants store
     const bool p16 = a.pg.log2_page == 4;
 #define X(DK, DV, REP)                                                  \
     if (!g.kv_f16 && g.dk == DK && g.dv == DV && g.rep == REP) {        \
         if (p16)                                                        \
-            launch_dec<DK, DV, REP, (DK + DV + 8 <= 128)>(a, waves, s); \
+            launch_dec<DK, DV, REP, (DK + DV + 8 <= 128)>(a, waves, f, s); \
         else                                                            \
-            launch_dec<DK, DV, REP, false>(a, waves, s);                \
+            launch_dec<DK, DV, REP, false>(a, waves, f, s);             \
         return hipGetLastError();                                       \
     }
     NDA_DEC_GEOMETRIES(X)
