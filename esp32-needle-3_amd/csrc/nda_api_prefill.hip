@@ -135,7 +135,10 @@ int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t 
     std::vector<std::array<uint32_t, 3>> bins[8];
     size_t items = 0;
     pl.n_items = 8 * (size_t)prefill_bins(c, nseq, ids, n_tokens, pl.rep, pl.trows, bins, &items);
-    if (!pl.valu)
+    // fp16 K/V only: an int8 prefill's weights carry the v scales, and its
+    // errors on keys with large scores (3e-5 against 64 bits, where fp16's are
+    // 1e-6) follow the order of the tiles
+    if (!pl.valu && c->geo.kv_f16)
         pl.ksplit = prefill_ksplit(c, items, pl.tab_cap, pl.waves);
     c->plan = pl;
     c->plan_key = std::move(key);
