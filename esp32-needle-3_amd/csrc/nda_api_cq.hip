@@ -247,11 +247,31 @@ int nda_cq_prepare_split(const nda_cq *t, uint32_t rows, const float *x, void *x
     return launch_cq_prepare_split(a, (hipStream_t)stream) == hipSuccess ? NDA_OK : NDA_ERR_HIP;
 }
 
-// The kernels of the split-precision GEMM: CQ_BIG cq_gemm_split_kernel,
-// CQ_FINE cq_gemm_fine_kernel, CQ_RAW cq_gemm_raw_kernel (xs then holds the
-// raw activations [rows][in], which it prepares itself; cq_raw_ok).
-enum CqForm { CQ_BIG, CQ_FINE, CQ_RAW };
-static int cq_gemm_split(const nda_cq *const *ts, uint32_t n, uint32_t rows, const void *xs, CqForm form,
+// Outputs per tile of a launch: 64 or 128 of cq_gemm_fine_kernel (over 64
+// rows), 0 the big kernel. The smaller tile up to one per CU (256), where a
+// launch is one work-group's walk whatever the tiles. The bits are the same.
+// us at 768 columns, 64 / 128 / big:
+//   q/k/v/gate (1568 outputs)  300 rows (125 tiles of 64) 9.3 / 12.3 / 20.5,
+//     600 (250) 10.4 / 13.2 / 20.8, 700 (275; 154 of 128) 16.1 / 13.5 / 20.9,
+//     1024 (224) 16.8 / 14.4 / 21.6, 1300 (294) 23.3 / 21.9 / 22.2, 2048 29.7
+//     / 23.8 / 23.8, 4096 51.8 / 41.9 / 37.5;
+//   out_proj (768 outputs)  300 rows 8.9 / 11.3 / 19.4, 1300 (252 of 64) 10.4
+//     / 12.6 / 20.2, 1400 (264; 132 of 128) 15.8 / 12.7 / 20.3, 2400 (228)
+//     18.0 / 15.1 / 21.4, 2700 (258) 23.3 / 21.6 / 21.2, 4096 25.1 / 22.5 / 22.9.
+static uint32_t cq_fine(const nda_cq *const *ts, uint32_t n, uint32_t rows)
+{
+    uint64_t t64 = 0, t128 = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        t64 += (ts[i]->out + 63) / 64;
+        t128 += (ts[i]->out + 127) / 128;
+    }
+    const uint64_t rt = (rows + 63ull) / 64;
+    return t64 * rt <= 256 ? 64 : t128 * rt <= 256 ? 128 : 0;
+}
+
+// raw: xs holds the raw activations [rows][in], which the kernel prepares
+// itself (cq_raw); the bits of ys are the same.
+static int cq_gemm_split(const nda_cq *const *ts, uint32_t n, uint32_t rows, const void *xs, bool raw,
                          float *const *ys, void *stream)
 {
     if (!ts || !ys || n == 0 || n > (uint32_t)CQ_MAX_T || (rows && !xs))
@@ -263,15 +283,13 @@ static int cq_gemm_split(const nda_cq *const *ts, uint32_t n, uint32_t rows, con
         return NDA_ERR_ARG;
     CqSplitArgs a{};
     a.xs = (const _Float16 *)xs;
-    a.rexp = form == CQ_RAW ? nullptr : (const int32_t *)(a.xs + split_rows(rows) * t0->in_pad * 2);
+    a.rexp = raw ? nullptr : (const int32_t *)(a.xs + split_rows(rows) * t0->in_pad * 2);
     a.x = (const float *)xs;
-    a.in = t0->in;
     a.scale = 1.0f / sqrtf((float)t0->group);
     a.rows = rows;
     a.in_pad = t0->in_pad;
     a.log2_group = (uint32_t)__builtin_ctz(t0->group);
     a.nt = n;
-    const uint32_t nt = form == CQ_BIG ? CQ_SPLIT_NT : CQ_FINE_NT;
     uint32_t tiles = 0;
     for (uint32_t i = 0; i < n; i++) {
         const nda_cq *t = ts[i];
@@ -286,40 +304,23 @@ static int cq_gemm_split(const nda_cq *const *ts, uint32_t n, uint32_t rows, con
         a.tab[i] = t->tab;
         a.cexp[i] = t->cexp;
         a.out[i] = t->out;
-        a.tile0[i] = tiles;
-        tiles += (t->out + nt - 1) / nt;
+        tiles += (t->out + CQ_SPLIT_NT - 1) / CQ_SPLIT_NT;
     }
-    a.tile0[n] = tiles;
-    if (tiles > 65535 * (CQ_SPLIT_NT / nt))
+    if (tiles > 65535)
         return NDA_ERR_ARG;
+    const uint32_t fine = raw ? 0 : cq_fine(ts, n, rows), nt = raw ? 128 : fine ? fine : CQ_SPLIT_NT;
+    for (uint32_t i = 0; i < n; i++)
+        a.tile0[i + 1] = a.tile0[i] + (a.out[i] + nt - 1) / nt;
     hipStream_t st = (hipStream_t)stream;
-    const hipError_t e = form == CQ_RAW ? launch_cq_gemm_raw(a, st)
-                         : form == CQ_FINE ? launch_cq_gemm_fine(a, st) : launch_cq_gemm_split(a, st);
+    const hipError_t e = raw ? launch_cq_gemm_raw(a, st)
+                         : fine ? launch_cq_gemm_fine(a, fine, st) : launch_cq_gemm_split(a, st);
     return e == hipSuccess ? NDA_OK : NDA_ERR_HIP;
 }
-
-// The big kernel's 128 x 128 tiles want most of the CUs busy: up to 160 of
-// them (of 256 CUs) the 64 x 64 tiles take over. At 768 columns, us, big ->
-// fine: q/k/v/gate (1568 outputs) 300 rows 20.6 -> 9.5, 1024 rows (104 tiles)
-// 21.8 -> 14.1, 2048 (208) 23.3 against 25.3, 4096 37.9 against 41.9; out_proj
-// (768 outputs) 1024 rows 20.4 -> 10.5, 2048 21.0 -> 13.8, 3000 (144) 22.1 ->
-// 20.4, 4096 (192) 22.9 against 23.1, 8192 39.5 against 42.4.
-static CqForm cq_form(const nda_cq *const *ts, uint32_t n, uint32_t rows)
-{
-    uint64_t tiles = 0;
-    for (uint32_t i = 0; i < n; i++)
-        tiles += (ts[i]->out + CQ_SPLIT_NT - 1) / CQ_SPLIT_NT;
-    return tiles * ((rows + (uint64_t)CQ_SPLIT_MT - 1) / CQ_SPLIT_MT) <= 160 ? CQ_FINE : CQ_BIG;
-}
-
-// The calls on prepared rows go by the rows alone, so that several tensors in
-// one launch equal their single launches bit for bit.
-constexpr uint32_t CQ_FINE_ROWS = 1024;
 
 int nda_cq_gemm_split_many(const nda_cq *const *ts, uint32_t n, uint32_t rows, const void *xs, float *const *ys,
                            void *stream)
 {
-    return cq_gemm_split(ts, n, rows, xs, rows <= CQ_FINE_ROWS ? CQ_FINE : CQ_BIG, ys, stream);
+    return cq_gemm_split(ts, n, rows, xs, false, ys, stream);
 }
 
 int nda_cq_gemm_split(const nda_cq *t, uint32_t rows, const void *xs, float *y, void *stream)
@@ -334,15 +335,21 @@ int nda_cq_gemm_split(const nda_cq *t, uint32_t rows, const void *xs, float *y, 
 // otherwise. xs holds nda_cq_split_bytes(ts[0], rows), at least the fp32
 // prepared form's rows * in_pad floats.
 constexpr uint32_t CQ_LUT_ROWS = 64;
-// Up to CQ_RAW_ROWS rows the split GEMM prepares its rows itself: a launch
-// less, against a transform per 64 outputs. At the archive's shape, us per
-// projection (prepare + GEMM -> raw; mean of q/k/v/gate and out_proj): 65 rows
-// 4.4 + 9.1 -> 11.1, 300 rows 4.3 + 10.9 -> 11.8, 512 rows 4.1 + 10.9 -> 15.8
-// (and the launch), 700 rows 4.9 + 12.4 -> 24.1.
-constexpr uint32_t CQ_RAW_ROWS = 512;
-static bool cq_raw_ok(const nda_cq *t)
+// One launch for the prepare and the split GEMM: group 128, whole groups, and
+// up to one work-group (32 rows x 128 outputs) per CU (256), where the
+// transform's repeats cost less than a launch. us per layer of the block at
+// the archive's shape, prepare + GEMM -> raw: 65 rows 34.2 -> 32.3, 300 36.2
+// -> 34.1, 600 (247 tiles of q/k/v/gate) 43.8 -> 41.9, 1024 (out_proj alone:
+// 192) 49.6 -> 45.6; beyond one per CU 640 rows (260 tiles) 44.1 -> 51.7.
+static bool cq_raw(const nda_cq *const *ts, uint32_t n, uint32_t rows)
 {
-    return t->group == 128 && t->in == t->in_pad && t->in_pad <= 128 * CQ_RAW_MAX_G;
+    const nda_cq *t0 = ts[0];
+    if (t0->group != 128 || t0->in != t0->in_pad || t0->in_pad > 128 * CQ_RAW_MAX_G)
+        return false;
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < n; i++)
+        tiles += (ts[i]->out + 127) / 128;
+    return tiles * ((rows + 31ull) / 32) <= 256;
 }
 static int cq_project(const nda_cq *const *ts, uint32_t n, uint32_t rows, const float *x, void *xs,
                       float *const *ys, hipStream_t st)
@@ -360,12 +367,12 @@ static int cq_project(const nda_cq *const *ts, uint32_t n, uint32_t rows, const 
             return rc;
         return cq_lut2(ts, n, rows, (const float *)xs, false, ys, st);
     }
-    if (split && rows <= CQ_RAW_ROWS && cq_raw_ok(ts[0]))
-        return cq_gemm_split(ts, n, rows, x, CQ_RAW, ys, st);
+    if (split && cq_raw(ts, n, rows))
+        return cq_gemm_split(ts, n, rows, x, true, ys, st);
     if (split) {
         if (int rc = nda_cq_prepare_split(ts[0], rows, x, xs, st))
             return rc;
-        return cq_gemm_split(ts, n, rows, xs, cq_form(ts, n, rows), ys, st);
+        return nda_cq_gemm_split_many(ts, n, rows, xs, ys, st);
     }
     if (int rc = nda_cq_prepare(ts[0], rows, x, (float *)xs, st))
         return rc;

@@ -814,132 +814,30 @@ void cq_gemm_split_kernel(CqSplitArgs a)
         drain();
 }
 
-// The split GEMM for batches that give cq_gemm_split_kernel too few of its
-// 128 x 128 tiles to fill the chip (or to balance it): a work-group is 64 x 64
-// outputs, its four waves each take a quarter of the columns (steps) of the
-// whole tile, and their sums meet in LDS in column order. A wave's step is the
-// big kernel's (2 x 2 blocks, 24 MFMAs), so the operand traffic per product
-// is the same; the tile is a quarter of the size and a quarter of the steps
-// long. 300 rows x 768 columns x 1568 outputs: 20.6 -> 9.5 us (1024 rows 21.8
-// -> 14.1, 0.5 PFLOP/s of MFMA). Four partial sums instead of one chain also
-// lower the error against 64 bits, 3.3e-7 -> 2.0e-7.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void cq_gemm_fine_kernel(CqSplitArgs a)
+// A wave's 32 rows x 32 OB outputs, scaled back by the row's and the column's
+// powers of two (rx: lane t row t's; ce: of the lane's outputs), through its
+// stage [32][32 OB + 4] (its LDS operations complete in order), then 16-byte
+// stores along the rows.
+template <int OB>
+__device__ __forceinline__ void store_block(float *sw, const float16v *acc, int rx, const int *ce, float *y,
+                                            uint32_t r0, uint32_t rows, uint32_t o0, uint32_t out, int lane)
 {
-    constexpr int SLD = 64 + 4;                         // row stride of a wave's stage, floats
-    __shared__ __attribute__((aligned(16))) float stage[4][64 * SLD];
-    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, jh = lane >> 5;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // work-group w runs on XCD w % 8, which walks a contiguous range of
-    // items: the output tiles of one row tile read its X rows from one L2
-    const uint32_t ntiles = a.tile0[a.nt], total = (a.rows + 63) / 64 * ntiles;
-    const uint32_t item = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
-    if (item >= total)
-        return;
-    const uint32_t r0 = item / ntiles * 64, tile = item % ntiles, ti = tensor_of(a.tile0, a.nt, tile);
-    const uint32_t out = a.out[ti], o0 = (tile - a.tile0[ti]) * 64;
-    const uint32_t nkb = a.in_pad / 16, nsteps = a.in_pad / CS_KT;
-    const uint32_t s0 = nsteps * wave / 4, s1 = nsteps * (wave + 1) / 4;
-
-    // rows or outputs past the end read row block 0 or output 0: what they
-    // feed is never stored
-    const half8 *xr[2];
-    uint32_t oc[2];
+    constexpr int SLD = 32 * OB + 4;
+    const int ln = lane & 31, jh = lane >> 5;
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
-        const uint32_t rb = r0 + 32 * b < a.rows ? (r0 >> 5) + b : 0, o = o0 + 32 * b + ln;
-        xr[b] = reinterpret_cast<const half8 *>(a.xs) + (uint64_t)rb * nkb * 128;
-        oc[b] = o < out ? o : 0;
+    for (int i = 0; i < 16; i++) {
+        const int t = 8 * (i >> 2) + 4 * jh + (i & 3), e = __shfl(rx, t, 64);
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            sw[t * SLD + 32 * ob + ln] = ldexpf(acc[ob][i], -(e + ce[ob]));
     }
-    struct Step {
-        half8 x[2][2][2];                               // [ks][rb][plane]
-        uint32_t cw[2];
-        uint4 tab[2];
-    };
-    auto load = [&](uint32_t s, Step &st) __attribute__((always_inline)) {
-        s = min(s, nsteps - 1);                         // (past the end: a step that exists, not used)
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-            for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-                for (int p = 0; p < 2; p++)
-                    st.x[ks][rb][p] = xr[rb][((2 * s + ks) * 2 + p) * 64 + lane];
-#pragma unroll
-        for (int ob = 0; ob < 2; ob++) {
-            st.cw[ob] = a.cw[ti][((uint64_t)s * out + oc[ob]) * 2 + jh];
-            st.tab[ob] = a.tab[ti][(uint64_t)((s * CS_KT) >> a.log2_group) * out + oc[ob]];
-        }
-    };
-    float16v acc[2][2];
-#pragma unroll
-    for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-        for (int ob = 0; ob < 2; ob++)
-            acc[rb][ob] = float16v{};
-    auto compute = [&](const Step &st) __attribute__((always_inline)) {
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-            half8 wa[2], wb[2];
-#pragma unroll
-            for (int ob = 0; ob < 2; ob++)
-                cq_decode8(st.tab[ob], st.cw[ob] >> (4 * ks), wa[ob], wb[ob]);
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.x[ks][q >> 1][0], wa[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.x[ks][q >> 1][1], wa[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.x[ks][q >> 1][0], wb[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
-        }
-    };
-    // two register sets in turn, loads a step ahead of the MFMAs (the
-    // scheduling barriers keep them there)
-    Step sa, sb;
-    if (s0 < s1)
-        load(s0, sa);
-    const int rx = a.rexp[min(r0 + lane, a.rows - 1)];  // lane t: row r0 + t
-    int ce[2];
-#pragma unroll
-    for (int ob = 0; ob < 2; ob++)
-        ce[ob] = a.cexp[ti][oc[ob]];
-    for (uint32_t s = s0; s < s1; s += 2) {
-        load(s + 1, sb);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(sa);
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + 1 >= s1)
-            break;
-        load(s + 2, sa);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(sb);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    float *const sw = stage[wave];
-#pragma unroll
-    for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = 32 * rb + 8 * (i >> 2) + 4 * jh + (i & 3);
-            const int e = __shfl(rx, t, 64);
-#pragma unroll
-            for (int ob = 0; ob < 2; ob++)
-                sw[t * SLD + 32 * ob + ln] = ldexpf(acc[rb][ob][i], -(e + ce[ob]));
-        }
-    __syncthreads();
-    float *y = a.y[ti];
+    __builtin_amdgcn_wave_barrier();
     const bool v4 = (out & 3u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
 #pragma unroll
-    for (uint32_t u = 0; u < 4; u++) {
-        const uint32_t r = 16 * u + tid / 16, c = 4 * (tid % 16), row = r0 + r, o = o0 + c;
-        const float *p = &stage[0][0] + r * SLD + c;
-        float4v z = *reinterpret_cast<const float4v *>(p);
-#pragma unroll
-        for (int w = 1; w < 4; w++)
-            z += *reinterpret_cast<const float4v *>(p + w * 64 * SLD);
-        if (row >= a.rows)
+    for (uint32_t u = 0; u < 4 * OB; u++) {
+        const uint32_t r = 8 / OB * u + lane / (8 * OB), c = 4 * (lane % (8 * OB)), row = r0 + r, o = o0 + c;
+        const float4v z = *reinterpret_cast<const float4v *>(sw + r * SLD + c);
+        if (row >= rows)
             continue;
         float *dst = y + (uint64_t)row * out + o;
         if (v4 && o + 3 < out) {
@@ -953,41 +851,158 @@ void cq_gemm_fine_kernel(CqSplitArgs a)
     }
 }
 
-// The split GEMM for a batch of some hundred rows, from the raw activations
-// (group 128): a work-group is 32 rows x 32 OB outputs, one wave per group of
-// 128 columns. Each wave loads its rows' group straight into the MFMA operand
-// layout (lane: row lane % 32, columns 16 kb + 8 (lane / 32) + [0, 8) of each
-// of 8 k-blocks), transforms it there - butterflies 1, 2, 4 inside a lane's
-// eight columns, 8 between the lane halves, 16, 32, 64 between k-blocks -
-// splits it into the fp16 pair at the (row, group)'s own power of two, and
-// multiplies it with the group's decoded weights. The groups' sums meet in
-// LDS in group order.
+// The split GEMM for batches that give cq_gemm_split_kernel too few of its
+// 128 x 128 tiles to fill the chip: a work-group is 64 rows x 64 OB outputs,
+// each wave 32 x 32 OB of them over all the columns. Every sum is the big
+// kernel's chain, product for product, so the results are the same bits and
+// which of the two ran shows in no stored code. A wave is independent of the
+// others (no barrier) and holds D steps of operands in a register ring.
 //
-// cq_gemm_split_kernel gives such a batch a few dozen work-groups that walk
-// all the columns in turn, behind a prepare launch. What bounds it
-// here is one wave's chain (loads, about 800 VALU of transform and split, 24
-// OB MFMAs); the transform is repeated for every 32 OB outputs, which is why
-// larger batches prepare their rows once. 300 rows, mean of q/k/v/gate and
-// out_proj: 5.2 + 21.2 us (prepare, big kernel) -> 11.8. A power of two per
-// (row, group) rather than per row: error against 64 bits 1.8e-7.
+// A launch of up to one work-group per CU is one wave's walk: 72 OB dependent
+// MFMAs a group of 128 columns, the next step's weights decoded between them;
+// past that, the operands through L1 (129 KB a wave at 768 columns and OB 1,
+// 64 bytes per cycle and CU), which OB 2 nearly halves per product. 300 rows x
+// 768 columns x 1568 outputs: 20.5 us in the big kernel, 9.3 here.
 template <int OB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void cq_gemm_fine_kernel(CqSplitArgs a)
+{
+    constexpr int NT = 32 * OB, SLD = NT + 4;           // a wave's outputs, row stride of its stage (floats)
+    constexpr int D = OB == 1 ? 8 : 5;
+    __shared__ __attribute__((aligned(16))) float stage[4][32 * SLD];
+    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, jh = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // work-group w runs on XCD w % 8, which walks a contiguous range of
+    // items: the output tiles of one row tile read its X rows from one L2
+    const uint32_t ntiles = a.tile0[a.nt], total = (a.rows + 63) / 64 * ntiles;
+    const uint32_t item = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+    if (item >= total)
+        return;
+    const uint32_t tile = item % ntiles, ti = tensor_of(a.tile0, a.nt, tile);
+    const uint32_t r0 = item / ntiles * 64 + 32 * (wave & 1);
+    const uint32_t out = a.out[ti], o0 = ((tile - a.tile0[ti]) * 2 + (wave >> 1)) * NT;
+    if (r0 >= a.rows || o0 >= out)
+        return;
+    const uint32_t nkb = a.in_pad / 16, nsteps = a.in_pad / CS_KT;
+
+    // outputs past the end read output 0: what they feed is never stored
+    const half8 *xr = reinterpret_cast<const half8 *>(a.xs) + (uint64_t)(r0 >> 5) * nkb * 128 + lane;
+    const uint32_t *cw[OB];
+    const uint4 *tab[OB];
+    int ce[OB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) {
+        const uint32_t o = o0 + 32 * ob + ln, oc = o < out ? o : 0;
+        cw[ob] = a.cw[ti] + (uint64_t)oc * 2 + jh;
+        tab[ob] = a.tab[ti] + oc;
+        ce[ob] = a.cexp[ti][oc];
+    }
+    const int rx = a.rexp[min(r0 + ln, a.rows - 1)];    // lane t: row r0 + t
+    struct Step {
+        half8 x[2][2];                                  // [ks][plane]
+        uint32_t cw[OB];
+        uint4 tab[OB];
+    };
+    auto load = [&](uint32_t s, Step &st) __attribute__((always_inline)) {
+        s = min(s, nsteps - 1);                         // (past the end: a step that exists, not used)
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+                st.x[ks][p] = xr[((2 * s + ks) * 2 + p) * 64];
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++) {
+            st.cw[ob] = cw[ob][(uint64_t)s * out * 2];
+            st.tab[ob] = tab[ob][(uint64_t)((s * CS_KT) >> a.log2_group) * out];
+        }
+    };
+    half8 wa[2][OB], wb[2][OB];                         // [ks][ob] the next step's weights
+    auto decode = [&](const Step &st, int ks) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+            cq_decode8(st.tab[ob], st.cw[ob] >> (4 * ks), wa[ks][ob], wb[ks][ob]);
+    };
+    Step ring[D];
+#pragma unroll
+    for (int k = 0; k < D - 1; k++)
+        load(k, ring[k]);
+    float16v acc[OB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+        acc[ob] = float16v{};
+    decode(ring[0], 0);
+    decode(ring[0], 1);
+    for (uint32_t s = 0; s < nsteps; s += D) {
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            if (s + k >= nsteps)
+                break;
+            // into the slot of the step before this one; the next step's
+            // weights are decoded between this step's MFMAs
+            load(s + k + D - 1, ring[(k + D - 1) % D]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                half8 va[OB], vb[OB];
+#pragma unroll
+                for (int ob = 0; ob < OB; ob++) {
+                    va[ob] = wa[ks][ob];
+                    vb[ob] = wb[ks][ob];
+                }
+                decode(ring[(k + 1) % D], ks);
+#pragma unroll
+                for (int ob = 0; ob < OB; ob++)
+                    acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ring[k].x[ks][0], va[ob], acc[ob], 0, 0, 0);
+#pragma unroll
+                for (int ob = 0; ob < OB; ob++)
+                    acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ring[k].x[ks][1], va[ob], acc[ob], 0, 0, 0);
+#pragma unroll
+                for (int ob = 0; ob < OB; ob++)
+                    acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ring[k].x[ks][0], vb[ob], acc[ob], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    store_block<OB>(stage[wave], acc, rx, ce, a.y[ti], r0, a.rows, o0, out, lane);
+}
+
+// The split GEMM for a batch of some hundred rows, from the raw activations
+// (group 128): a work-group is 32 rows x 128 outputs, and prepares its rows
+// itself, one wave per group of 128 columns. Each wave loads its rows' group
+// straight into the MFMA operand layout (lane: row lane % 32, columns 16 kb +
+// 8 (lane / 32) + [0, 8) of each of 8 k-blocks), transforms it there -
+// butterflies 1, 2, 4 inside a lane's eight columns, 8 between the lane
+// halves, 16, 32, 64 between k-blocks - finds the row's largest value with
+// the other waves', splits its values into the fp16 pair at the row's power
+// of two and leaves the operands in LDS, where four waves take them up, each
+// for 32 outputs over all the columns. Every step rounds as the prepare and
+// cq_gemm_split_kernel do, so the results are the same bits.
+//
+// What bounds it is one work-group's walk: loads, about 800 VALU of transform
+// and split a wave, then 144 dependent MFMAs at 768 columns (a sum per group,
+// side by side, takes 5 us less per layer of the block at 300 rows, but rounds
+// differently, so stored codes would follow the batch's size). 300 rows x 768
+// columns, q/k/v/gate and out_proj with what lies between them: 36.2 us a
+// layer with the prepare as a launch of its own, 34.1 here.
 __global__ __launch_bounds__(64 * CQ_RAW_MAX_G)
 void cq_gemm_raw_kernel(CqSplitArgs a)
 {
 #pragma clang fp contract(off)
-    constexpr int SLD = 32 * OB + 4;                    // row stride of a wave's stage, floats
-    extern __shared__ __attribute__((aligned(16))) float raw_stage[];   // [groups][32][SLD]
+    constexpr int SLD = 32 + 4, D = 8;                  // row stride of a wave's stage, floats; weights in flight, steps
+    extern __shared__ __attribute__((aligned(16))) half8 raw_x[];       // [k-block][plane][lane]
+    __shared__ float rmax[CQ_RAW_MAX_G][32];
+    __shared__ __attribute__((aligned(16))) float stage[4][32 * SLD];
     const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, jh = lane >> 5;
-    const uint32_t g = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), ng = a.in_pad / 128, nsteps = 4 * ng;
     const uint32_t tile = blockIdx.x, r0 = blockIdx.y * 32, ti = tensor_of(a.tile0, a.nt, tile);
-    const uint32_t out = a.out[ti], o0 = (tile - a.tile0[ti]) * (32 * OB);
+    const uint32_t out = a.out[ti], o0 = (tile - a.tile0[ti]) * 128 + 32 * wave;
+    const bool mult = wave < 4 && o0 < out;
 
-    // every load first (the scheduler otherwise leaves the weights' pointers,
-    // and so their loads, behind the transform); rows and outputs past the
-    // end read the last row and output 0: what they feed is never stored
+    // every load first; rows and outputs past the end read the last row and
+    // output 0: what they feed is never stored
     float v[8][8];
-    {
-        const float *x = a.x + (uint64_t)min(r0 + ln, a.rows - 1) * a.in + g * 128 + 8 * jh;
+    if (wave < ng) {
+        const float *x = a.x + (uint64_t)min(r0 + ln, a.rows - 1) * a.in_pad + wave * 128 + 8 * jh;
 #pragma unroll
         for (int kb = 0; kb < 8; kb++) {
             const float4 u0 = *reinterpret_cast<const float4 *>(x + 16 * kb);
@@ -1002,148 +1017,142 @@ void cq_gemm_raw_kernel(CqSplitArgs a)
             v[kb][7] = u1.w;
         }
     }
-    uint32_t cw[4][OB];
-    uint4 tab[OB];
-    int32_t ce[OB];
+    const uint32_t oc = mult && o0 + ln < out ? o0 + ln : 0;
+    const uint32_t *cw = a.cw[ti] + (uint64_t)oc * 2 + jh;
+    const uint4 *tab = a.tab[ti] + oc;
+    struct Step {
+        uint32_t cw;
+        uint4 tab;
+    };
+    auto load = [&](uint32_t s, Step &st) __attribute__((always_inline)) {
+        s = min(s, nsteps - 1);                         // (past the end: a step that exists, not used)
+        st.cw = cw[(uint64_t)s * out * 2];
+        st.tab = tab[(uint64_t)(s >> 2) * out];
+    };
+    Step ring[D];
 #pragma unroll
-    for (int ob = 0; ob < OB; ob++) {
-        const uint32_t o = o0 + 32 * ob + ln, oc = o < out ? o : 0;
-#pragma unroll
-        for (int s = 0; s < 4; s++)
-            cw[s][ob] = a.cw[ti][((uint64_t)(4 * g + s) * out + oc) * 2 + jh];
-        tab[ob] = a.tab[ti][(uint64_t)g * out + oc];
-        ce[ob] = a.cexp[ti][oc];
-    }
+    for (int k = 0; k < D - 1; k++)
+        load(k, ring[k]);
+    const int ce = a.cexp[ti][oc];
     __builtin_amdgcn_sched_barrier(0);
 
-    // the engine's butterflies, stage by stage
+    if (wave < ng) {
+        // the engine's butterflies, stage by stage
 #pragma unroll
-    for (int len = 1; len < 8; len <<= 1)
+        for (int len = 1; len < 8; len <<= 1)
+#pragma unroll
+            for (int kb = 0; kb < 8; kb++)
+#pragma unroll
+                for (int s = 0; s < 8; s++)
+                    if ((s & len) == 0) {
+                        const float u = v[kb][s], w = v[kb][s + len];
+                        v[kb][s] = u + w;
+                        v[kb][s + len] = u - w;
+                    }
+        // length 8, two values at a time: one swap brings (p of both halves)
+        // into the lower lanes and (q of both) into the upper ones, one takes
+        // the sums and differences back
+#pragma unroll
+        for (int kb = 0; kb < 8; kb++)
+#pragma unroll
+            for (int s = 0; s < 8; s += 2) {
+                const auto f = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[kb][s]), __float_as_uint(v[kb][s + 1]),
+                                                                false, false);
+                const float lo = __uint_as_float(f[0]), hi = __uint_as_float(f[1]);
+                const float sum = lo + hi, dif = lo - hi;
+                const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(dif), false, false);
+                v[kb][s] = __uint_as_float(b[0]);
+                v[kb][s + 1] = __uint_as_float(b[1]);
+            }
+#pragma unroll
+        for (int len = 1; len < 8; len <<= 1)
+#pragma unroll
+            for (int kb = 0; kb < 8; kb++)
+                if ((kb & len) == 0)
+#pragma unroll
+                    for (int s = 0; s < 8; s++) {
+                        const float u = v[kb][s], w = v[kb + len][s];
+                        v[kb][s] = u + w;
+                        v[kb + len][s] = u - w;
+                    }
+        float mx = 0.0f;
 #pragma unroll
         for (int kb = 0; kb < 8; kb++)
 #pragma unroll
-            for (int s = 0; s < 8; s++)
-                if ((s & len) == 0) {
-                    const float u = v[kb][s], w = v[kb][s + len];
-                    v[kb][s] = u + w;
-                    v[kb][s + len] = u - w;
-                }
-    // length 8, two values at a time: one swap brings (p of both halves) into
-    // the lower lanes and (q of both) into the upper ones, one takes the sums
-    // and differences back
-#pragma unroll
-    for (int kb = 0; kb < 8; kb++)
-#pragma unroll
-        for (int s = 0; s < 8; s += 2) {
-            const auto f = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[kb][s]), __float_as_uint(v[kb][s + 1]),
-                                                            false, false);
-            const float lo = __uint_as_float(f[0]), hi = __uint_as_float(f[1]);
-            const float sum = lo + hi, dif = lo - hi;
-            const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(dif), false, false);
-            v[kb][s] = __uint_as_float(b[0]);
-            v[kb][s + 1] = __uint_as_float(b[1]);
-        }
-#pragma unroll
-    for (int len = 1; len < 8; len <<= 1)
-#pragma unroll
-        for (int kb = 0; kb < 8; kb++)
-            if ((kb & len) == 0)
-#pragma unroll
-                for (int s = 0; s < 8; s++) {
-                    const float u = v[kb][s], w = v[kb + len][s];
-                    v[kb][s] = u + w;
-                    v[kb + len][s] = u - w;
-                }
-
-    // this (row, group)'s power of two, then the pairs
+            for (int s = 0; s < 8; s++) {
+                v[kb][s] *= a.scale;                    // the engine's prepared value
+                mx = fmaxf(mx, fabsf(v[kb][s]));
+            }
+        mx = fmaxf(mx, xor_lanes<32>(mx, lane));
+        if (jh == 0)
+            rmax[wave][ln] = mx;
+    }
+    __syncthreads();
+    // row r0 + ln's power of two
     float mx = 0.0f;
-#pragma unroll
-    for (int kb = 0; kb < 8; kb++)
-#pragma unroll
-        for (int s = 0; s < 8; s++)
-            mx = fmaxf(mx, fabsf(v[kb][s]));
-    mx = fmaxf(mx, xor_lanes<32>(mx, lane)) * a.scale;
+    for (uint32_t g = 0; g < ng; g++)
+        mx = fmaxf(mx, rmax[g][ln]);
     int e = 0, sh = 0;
     if (mx > 0.0f && mx <= FLT_MAX) {
         (void)frexpf(mx, &e);
         sh = 15 - e;                                    // mx * 2^sh in [2^14, 2^15)
     }
-    // the engine's prepared value (one rounding) times 2^sh in one product:
-    // scale * 2^sh is exact up to 2^120, and the rare larger rest (a group
-    // below 2^-105) exact again
-    const float f = ldexpf(a.scale, min(sh, 120)), rest = ldexpf(1.0f, max(sh - 120, 0));
-    const bool tiny = __ballot(sh > 120) != 0;
-    half8 xa[8], xb[8];
-    const float neg1 = opaque_neg1();
+    if (wave < ng) {
+        const float neg1 = opaque_neg1();
 #pragma unroll
-    for (int kb = 0; kb < 8; kb++) {
-        u32x4 ha, hb;
+        for (int kb = 0; kb < 8; kb++) {
+            u32x4 ha, hb;
 #pragma unroll
-        for (int s = 0; s < 8; s += 2) {
-            float y0 = v[kb][s] * f, y1 = v[kb][s + 1] * f;
-            if (tiny) {
-                y0 *= rest;
-                y1 *= rest;
+            for (int s = 0; s < 8; s += 2) {
+                float y0 = ldexpf(v[kb][s], sh), y1 = ldexpf(v[kb][s + 1], sh);
+                asm volatile("" : "+v"(y0), "+v"(y1));  // both halves from this one value
+                ha[s >> 1] = __builtin_bit_cast(uint32_t, half2v{(_Float16)y0, (_Float16)y1});
+                hb[s >> 1] = split_lo2(ha[s >> 1], y0, y1, neg1);
             }
-            asm volatile("" : "+v"(y0), "+v"(y1));      // both halves from this one value
-            ha[s >> 1] = __builtin_bit_cast(uint32_t, half2v{(_Float16)y0, (_Float16)y1});
-            hb[s >> 1] = split_lo2(ha[s >> 1], y0, y1, neg1);
+            raw_x[((8 * wave + kb) * 2 + 0) * 64 + lane] = __builtin_bit_cast(half8, ha);
+            raw_x[((8 * wave + kb) * 2 + 1) * 64 + lane] = __builtin_bit_cast(half8, hb);
         }
-        xa[kb] = __builtin_bit_cast(half8, ha);
-        xb[kb] = __builtin_bit_cast(half8, hb);
-    }
-
-    float16v acc[OB];
-#pragma unroll
-    for (int ob = 0; ob < OB; ob++)
-        acc[ob] = float16v{};
-#pragma unroll
-    for (int kb = 0; kb < 8; kb++) {
-        half8 wa[OB], wb[OB];
-#pragma unroll
-        for (int ob = 0; ob < OB; ob++)
-            cq_decode8(tab[ob], cw[kb >> 1][ob] >> (4 * (kb & 1)), wa[ob], wb[ob]);
-#pragma unroll
-        for (int ob = 0; ob < OB; ob++)
-            acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[kb], wa[ob], acc[ob], 0, 0, 0);
-#pragma unroll
-        for (int ob = 0; ob < OB; ob++)
-            acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xb[kb], wa[ob], acc[ob], 0, 0, 0);
-#pragma unroll
-        for (int ob = 0; ob < OB; ob++)
-            acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[kb], wb[ob], acc[ob], 0, 0, 0);
-    }
-    float *const sw = raw_stage + g * 32 * SLD;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int t = 8 * (i >> 2) + 4 * jh + (i & 3);
-        const int rx = __shfl(sh, t, 64);               // row t's (both halves hold it)
-#pragma unroll
-        for (int ob = 0; ob < OB; ob++)
-            sw[t * SLD + 32 * ob + ln] = ldexpf(acc[ob][i], -(rx + ce[ob]));
     }
     __syncthreads();
-    const uint32_t ng = blockDim.x >> 6;
-    float *y = a.y[ti];
-    const bool v4 = (out & 3u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    for (uint32_t u = tid; u < 32 * 8 * OB; u += blockDim.x) {
-        const uint32_t r = u / (8 * OB), c = 4 * (u % (8 * OB)), row = r0 + r, o = o0 + c;
-        const float *p = raw_stage + r * SLD + c;
-        float4v z = *reinterpret_cast<const float4v *>(p);
-        for (uint32_t k = 1; k < ng; k++)
-            z += *reinterpret_cast<const float4v *>(p + k * 32 * SLD);
-        if (row >= a.rows)
-            continue;
-        float *dst = y + (uint64_t)row * out + o;
-        if (v4 && o + 3 < out) {
-            *reinterpret_cast<float4v *>(dst) = z;
-        } else {
+    if (!mult)
+        return;
+
+    // cq_gemm_fine_kernel's walk, the rows' operands read from LDS a step ahead
+    half8 x[2][2][2], wa[2], wb[2];                     // x: [step % 2][ks][plane]
+    auto rows_of = [&](uint32_t s, half8 (&d)[2][2]) __attribute__((always_inline)) {
+        s = min(s, nsteps - 1);
 #pragma unroll
-            for (uint32_t k = 0; k < 4; k++)
-                if (o + k < out)
-                    dst[k] = z[k];
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+                d[ks][p] = raw_x[((2 * s + ks) * 2 + p) * 64 + lane];
+    };
+    float16v acc = {};
+    rows_of(0, x[0]);
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+        cq_decode8(ring[0].tab, ring[0].cw >> (4 * ks), wa[ks], wb[ks]);
+    for (uint32_t s = 0; s < nsteps; s += D) {
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            if (s + k >= nsteps)
+                break;
+            load(s + k + D - 1, ring[(k + D - 1) % D]);
+            rows_of(s + k + 1, x[(k + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                const half8 va = wa[ks], vb = wb[ks];
+                const Step &nx = ring[(k + 1) % D];
+                cq_decode8(nx.tab, nx.cw >> (4 * ks), wa[ks], wb[ks]);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[k & 1][ks][0], va, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[k & 1][ks][1], va, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[k & 1][ks][0], vb, acc, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
+    store_block<1>(stage[wave], &acc, sh, &ce, a.y[ti], r0, a.rows, o0, out, lane);
 }
 
 // ------------------------------------------------ the engine's LUT order
@@ -1358,14 +1367,18 @@ hipError_t launch_cq_gemm_split(const CqSplitArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_cq_gemm_fine(const CqSplitArgs &a, hipStream_t s)
+hipError_t launch_cq_gemm_fine(const CqSplitArgs &a, uint32_t outs, hipStream_t s)
 {
     if (a.rows == 0 || a.nt == 0 || a.tile0[a.nt] == 0)
         return hipSuccess;
     const uint64_t items = (uint64_t)((a.rows + 63) / 64) * a.tile0[a.nt];
     if (items > 0x7FFFFFF0ull)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(cq_gemm_fine_kernel, dim3((uint32_t)((items + 7) / 8 * 8)), dim3(256), 0, s, a);
+    const dim3 grid((uint32_t)((items + 7) / 8 * 8));
+    if (outs == 64)
+        hipLaunchKernelGGL(cq_gemm_fine_kernel<1>, grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(cq_gemm_fine_kernel<2>, grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -1373,12 +1386,11 @@ hipError_t launch_cq_gemm_raw(const CqSplitArgs &a, hipStream_t s)
 {
     if (a.rows == 0 || a.nt == 0 || a.tile0[a.nt] == 0)
         return hipSuccess;
-    constexpr int OB = CQ_FINE_NT / 32;
     const uint32_t ng = a.in_pad / 128;
-    if (a.log2_group != 7 || a.in != a.in_pad || ng == 0 || ng > CQ_RAW_MAX_G || (a.rows + 31) / 32 > 65535)
+    if (a.log2_group != 7 || ng == 0 || ng > CQ_RAW_MAX_G || (a.rows + 31) / 32 > 65535)
         return hipErrorInvalidValue;
-    const size_t lds = (size_t)ng * 32 * (32 * OB + 4) * sizeof(float);
-    hipLaunchKernelGGL(cq_gemm_raw_kernel<OB>, dim3(a.tile0[a.nt], (a.rows + 31) / 32), dim3(64 * ng), lds, s, a);
+    hipLaunchKernelGGL(cq_gemm_raw_kernel, dim3(a.tile0[a.nt], (a.rows + 31) / 32), dim3(64 * std::max(4u, ng)),
+                       (size_t)ng * 16 * 64 * sizeof(half8), s, a);
     return hipGetLastError();
 }
 

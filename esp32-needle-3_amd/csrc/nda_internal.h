@@ -229,12 +229,11 @@ struct CqSplitArgs {
     const uint4 *tab[CQ_MAX_T];
     const int32_t *cexp[CQ_MAX_T];
     uint32_t out[CQ_MAX_T];
-    uint32_t tile0[CQ_MAX_T + 1];       /* first tile per tensor (of CQ_SPLIT_NT outputs; fine and raw: CQ_FINE_NT) */
+    uint32_t tile0[CQ_MAX_T + 1];       /* first tile per tensor (of CQ_SPLIT_NT outputs; fine: of its outs; raw: of 128) */
     uint32_t nt;
     uint32_t rows, in_pad, log2_group;
-    const float *x;                     /* cq_gemm_raw_kernel: the raw rows [rows][in] (xs, rexp unused), */
-    uint32_t in;                        /*   their width, and 1 / sqrt(group) */
-    float scale;
+    const float *x;                     /* cq_gemm_raw_kernel: the raw rows [rows][in_pad] (xs, rexp unused), */
+    float scale;                        /*   and 1 / sqrt(group) */
 };
 /* One 2-bit tensor's decode data for the split GEMM, built at creation:
  * cw [in_pad / 32][out][2] words, tab [ngroup][out] uint4, cexp [out]. */
@@ -253,7 +252,6 @@ struct CqTabArgs {
 constexpr int CQ_SPLIT_MT = 128;        /* rows per work-group */
 constexpr int CQ_SPLIT_OB = NDA_CQ_OB;  /* 32-output blocks per wave */
 constexpr int CQ_SPLIT_NT = 64 * CQ_SPLIT_OB;   /* outputs per work-group */
-constexpr int CQ_FINE_NT = 64;          /* cq_gemm_fine_kernel, cq_gemm_raw_kernel: outputs per work-group */
 constexpr uint32_t CQ_RAW_MAX_G = 8;    /* cq_gemm_raw_kernel: groups (of 128 columns), one per wave */
 
 hipError_t launch_cq_prepare(const CqPrepArgs &a, hipStream_t s);
@@ -262,9 +260,9 @@ hipError_t launch_cq_gemm(const CqGemmArgs &a, hipStream_t s);
 hipError_t launch_cq_lut2(const CqGemmArgs &a, bool prep, hipStream_t s);
 hipError_t launch_cq_prepare_split(const CqPrepSplitArgs &a, hipStream_t s);
 hipError_t launch_cq_gemm_split(const CqSplitArgs &a, hipStream_t s);
-/* the same from smaller tiles, for fewer rows */
-hipError_t launch_cq_gemm_fine(const CqSplitArgs &a, hipStream_t s);
-/* from raw rows: group 128, whole groups (in == in_pad), at most CQ_RAW_MAX_G */
+/* the same bits from smaller tiles, for fewer rows: 64 rows x outs (64 or 128) */
+hipError_t launch_cq_gemm_fine(const CqSplitArgs &a, uint32_t outs, hipStream_t s);
+/* the same bits from raw rows: group 128, whole groups (in == in_pad), at most CQ_RAW_MAX_G */
 hipError_t launch_cq_gemm_raw(const CqSplitArgs &a, hipStream_t s);
 hipError_t launch_cq_split_tables(const CqTabArgs &a, hipStream_t s);
 

@@ -379,13 +379,12 @@ def test_cq_split_persistent_walks_and_column_scales():
 
 
 @pytest.mark.parametrize("shape,rows", [
-    ((70, 32, 32, 2), 1), ((64, 64, 64, 2), 64), ((130, 96, 32, 2), 65),    # one to three steps for four waves
+    ((70, 32, 32, 2), 1), ((64, 64, 64, 2), 64), ((130, 96, 32, 2), 65),    # one to three steps of the operand ring
     ((65, 768, 128, 2), 63), ((96, 640, 128, 2), 129), ((200, 2048, 256, 2), 1023),
-    ((33, 768, 128, 2), 1024), ((33, 768, 128, 2), 1025),                   # the last row count of its kernel, the next's first
+    ((33, 768, 128, 2), 1024), ((33, 768, 128, 2), 1025),
 ])
 def test_cq_split_tiles(shape, rows):
-    """Edges of the 64 x 64 tiles and of the columns' split over four waves,
-    against the product in 64 bits of the prepared rows. Three fp16 products
+    """Edges of the small tiles, against the product in 64 bits of the prepared rows. Three fp16 products
     hold each term to about 2^-22 of itself and the sums round in fp32: at
     most (columns + 8) * 2^-24 of sum |w x|."""
     out, inp, group, b = shape
@@ -398,3 +397,33 @@ def test_cq_split_tiles(shape, rows):
         xh = O.cq_prepare(t, x[r]).astype(np.float64)
         err = np.abs(y[r].astype(np.float64) - w @ xh) / (np.abs(w) @ np.abs(xh))
         assert err.max() <= (t.in_pad + 8) * 2.0 ** -24, (r, float(err.max()))
+
+
+@pytest.mark.parametrize("inp,group", [(768, 128), (160, 32)])
+def test_cq_split_bits_do_not_follow_the_tile(inp, group):
+    """A row's product is the same bits in a launch of any number of rows and
+    tensors: 64 x 64, 64 x 128 and 128 x 128 tiles run the same chain of
+    products (64 rows, 700 and 1300 of 1568 outputs in one launch; each
+    tensor alone)."""
+    N = nda()
+    say("cq split bits", inp, group)
+    ts = [make_cq_tensor(500 + o, o, inp, group, 2) for o in (576, 96, 128, 768)]
+    qs = [N.CQ(t.out, t.inp, t.group, t.bits, t.blob, t.cb()) for t in ts]
+    x = np.random.default_rng(inp).standard_normal((1300, inp)).astype(np.float32)
+    want = None
+    for rows in (1300, 700, 64, 33):
+        xs = N.DevBuf(qs[0].split_bytes(rows))
+        qs[0].prepare_split(rows, N.DevBuf.from_array(x[:rows]), xs)
+        ys = [N.DevBuf(rows * t.out * 4) for t in ts]
+        N.cq_gemm_split_many(qs, rows, xs, ys)
+        N.device_sync()
+        got = [y.to_array(np.uint32, (rows, t.out)) for y, t in zip(ys, ts)]
+        for q, y, t, g in zip(qs, ys, ts, got):
+            q.gemm_split(rows, xs, y)
+            N.device_sync()
+            assert np.array_equal(y.to_array(np.uint32, (rows, t.out)), g), (rows, t.out)
+        want = want or got
+        for a, b, t in zip(got, want, ts):
+            assert np.array_equal(a, b[:rows]), (rows, t.out)
+    for q in qs:
+        q.close()
