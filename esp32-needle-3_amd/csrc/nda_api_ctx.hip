@@ -377,7 +377,7 @@ int upload_rows(nda_ctx *c, uint32_t rows, const uint32_t *row_seq, const uint32
     int rc = ensure_rows(c, rows);
     if (rc)
         return rc;
-    c->rows_list.what.clear();
+    c->rows_list.take(capturing(st));
     if (row_seq) {
         if (int rc2 = upload(c, c->d_rows, row_seq, rows * sizeof(uint32_t), st))
             return rc2;

@@ -17,9 +17,12 @@ namespace nda_host {
 // launch. Built once per change of sequence state (the 8 layers of a step
 // share it) and uploaded on the caller's stream; any permutation of the rows
 // gives the same results, so a stale order only costs time. A failed
-// allocation just leaves the rows in order.
+// allocation just leaves the rows in order, and so does a stream under
+// capture: its replays would read the order of whatever batch came last.
 static const uint32_t *decode_order(nda_ctx *c, uint32_t rows, hipStream_t st)
 {
+    if (capturing(st))
+        return nullptr;
     if (c->d_order && c->order_rows == rows && c->order_ver == c->state_ver)
         return c->d_order;
     std::vector<uint32_t> tiles(rows), first;
@@ -283,7 +286,7 @@ static int prefix_pass(nda_ctx *c, const AttnArgs &a, uint32_t nseq, const uint3
     // the list a step's first layer uploaded serves the others (it is made
     // of these values alone)
     const std::vector<uint32_t> key = {LIST_PREFIX_PASS, seq0, nseq, ps.n_sh, (uint32_t)ps.prefix};
-    if (!c->pf_list.holds(key, c->pf_cap, st)) {
+    if (capturing(st) || !c->pf_list.holds(key, c->pf_cap)) {
         std::vector<uint32_t> items;
         items.reserve(8 * (size_t)ps.n_items);
         for (uint32_t g = 0; g < c->cfg.n_kv_heads; g++)
@@ -298,10 +301,10 @@ static int prefix_pass(nda_ctx *c, const AttnArgs &a, uint32_t nseq, const uint3
             const uint32_t pad[8] = {0xFFFFFFFFu, 0, 0, 0, 0, 0, 0, 0};
             items.insert(items.end(), pad, pad + 8);
         }
-        c->pf_list.what.clear();
+        c->pf_list.take(capturing(st));
         if (int rc = upload(c, c->d_pf, items.data(), items.size() * 4, st))
             return rc;
-        c->pf_list.set(key, c->pf_cap, st);
+        c->pf_list.set(key, c->pf_cap);
     }
     PrefillArgs pa{};
     pa.q = a.q;

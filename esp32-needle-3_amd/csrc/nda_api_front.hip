@@ -197,7 +197,7 @@ int nda_front(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, co
     if (int rc = ensure_buf(c, c->d_front_rows, c->front_rows_cap, 3 * rows))
         return rc;
     const std::vector<uint32_t> key = list_key(LIST_FRONT, nseq, ids, n_tokens);
-    if (!c->front_list.holds(key, c->front_rows_cap, st)) {
+    if (capturing(st) || !c->front_list.holds(key, c->front_rows_cap)) {
         std::vector<uint32_t> host(3 * rows);
         for (uint32_t b = 0, r = 0; b < nseq; b++) {
             const uint32_t n = n_tokens ? n_tokens[b] : 1u;
@@ -207,10 +207,10 @@ int nda_front(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, co
                 host[2 * rows + r] = n;
             }
         }
-        c->front_list.what.clear();
+        c->front_list.take(capturing(st));
         if (int rc = upload(c, c->d_front_rows, host.data(), host.size() * 4, st))
             return rc;
-        c->front_list.set(key, c->front_rows_cap, st);
+        c->front_list.set(key, c->front_rows_cap);
     }
     FrontArgs a = front_args(c, layer);
     a.q = q;

@@ -216,7 +216,7 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
         return rc;
     const uint32_t *d_seq = c->d_rows, *d_t = c->d_rows + rows;
     const std::vector<uint32_t> rows_key = list_key(LIST_ROWS, nseq, ids, n_tokens);
-    if (!c->rows_list.holds(rows_key, c->rows_cap, st)) {
+    if (capturing(st) || !c->rows_list.holds(rows_key, c->rows_cap)) {
         std::vector<uint32_t> rseq(rows), rt(rows);
         for (uint32_t b = 0, r = 0; b < nseq; b++)
             for (uint32_t t = 0; t < n_tokens[b]; t++, r++) {
@@ -225,7 +225,7 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
             }
         if (int rc = upload_rows(c, (uint32_t)rows, rseq.data(), rt.data(), st, &d_seq, &d_t))
             return rc;
-        c->rows_list.set(rows_key, c->rows_cap, st);
+        c->rows_list.set(rows_key, c->rows_cap);
     }
     {
         AppendArgs a{};
@@ -258,7 +258,7 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
     // Of the plan alone, so a step's other layers take the list as it is.
     const std::vector<uint32_t> key = list_key(LIST_ITEMS, nseq, ids, n_tokens,
                                                {(uint32_t)c->state_ver, (uint32_t)(c->state_ver >> 32)});
-    if (!c->pf_list.holds(key, c->pf_cap, st)) {
+    if (capturing(st) || !c->pf_list.holds(key, c->pf_cap)) {
         std::vector<uint32_t> tok0(nseq);
         for (uint32_t b = 0, tok = 0; b < nseq; b++) {
             tok0[b] = tok;
@@ -283,10 +283,10 @@ int nda_prefill(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, 
         }
         if (items.size() != 8 * pl.n_items)
             return fail(c, NDA_ERR_STATE, "prefill work list: size differs from its plan");
-        c->pf_list.what.clear();
+        c->pf_list.take(capturing(st));
         if (int rc = upload(c, c->d_pf, items.data(), items.size() * 4, st))
             return rc;
-        c->pf_list.set(key, c->pf_cap, st);
+        c->pf_list.set(key, c->pf_cap);
     }
     PrefillArgs pa{};
     pa.q = q;

@@ -55,28 +55,8 @@ struct PrefillPlan {
     uint32_t ksplit = 0;                // parts per item's key tiles (0: whole)
 };
 
-// A list in a device buffer that several calls use: `what` it was built from
-// (its kind first, then the values), and the buffer's capacity, which grows
-// whenever the buffer is replaced. Empty: the buffer holds something else. A
-// stream being captured neither takes a list as held nor leaves one: the
-// graph's replays bring their own.
+// Whether a stream is under capture (or cannot be asked).
 bool capturing(hipStream_t st);
-struct DevList {
-    std::vector<uint32_t> what;
-    size_t cap = 0;
-    bool holds(const std::vector<uint32_t> &w, size_t c, hipStream_t st) const
-    {
-        return cap == c && what == w && !capturing(st);
-    }
-    void set(const std::vector<uint32_t> &w, size_t c, hipStream_t st)
-    {
-        what.clear();
-        if (!capturing(st)) {
-            what = w;
-            cap = c;
-        }
-    }
-};
 
 constexpr size_t UPLOAD_RING_BYTES = 16u << 20;
 constexpr int UPLOAD_EVENTS = 256;

@@ -33,6 +33,29 @@ struct SeqHost {
     uint32_t ring_lo = 0;      // ring positions in [n_sink, ring_lo) were overwritten before a rewind
 };
 
+// A list in a device buffer that several calls use: `what` it was built from
+// (its kind first, then the values), and the buffer's capacity, which grows
+// whenever the buffer is replaced. Empty: the buffer holds something else.
+// Every upload into the buffer is announced by take(). One under stream
+// capture becomes a copy in the graph, which each replay repeats unseen by the
+// host, so from then on nothing is taken as held.
+struct DevList {
+    std::vector<uint32_t> what;
+    size_t cap = 0;
+    bool in_graph = false;
+    bool holds(const std::vector<uint32_t> &w, size_t c) const { return !in_graph && cap == c && what == w; }
+    void take(bool captured)
+    {
+        what.clear();
+        in_graph |= captured;
+    }
+    void set(const std::vector<uint32_t> &w, size_t c)
+    {
+        what = w;
+        cap = c;
+    }
+};
+
 // nd_model_set_sink's clamp: at least ND_MIN_RECENT ring slots stay
 // (engine/src/nd_model.c:1314-1321).
 inline uint32_t clamp_sink(uint32_t window, uint32_t n)

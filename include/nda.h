@@ -23,7 +23,15 @@
  *     stream wait for the work queued on the previous one, so that stream
  *     must still exist then (nda_sync on it releases that). The inspection
  *     calls (nda_kv_read / nda_kv_write) run on the null stream the same way.
- *     Contexts do not order each other.
+ *     Contexts do not order each other;
+ *   - stream capture: a call under capture records its uploads (seq_ids,
+ *     n_tokens and the lists made of them; sequence state and page tables
+ *     that changed since the last launch) as copies from staging memory that
+ *     later calls reuse. Capture only calls that upload nothing - nda_decode,
+ *     nda_step, nda_attention and nda_attention_block of sequences 0..n-1,
+ *     after a first call outside the capture at the same positions - and
+ *     replay only while the context's buffers have not grown. A call outside
+ *     the graph is right whatever was captured and replayed before it.
  */
 #ifndef NDA_H
 #define NDA_H

@@ -281,9 +281,52 @@ static void check_oracle(std::mt19937 &rng)
     CHECK(out1 == out8);
 }
 
+// A list kept in a device buffer against a model of the buffer: calls in any
+// order, some under capture, whose copies replays repeat at any later time. A
+// list may be taken as held only if the buffer holds it.
+static void check_lists(std::mt19937 &rng)
+{
+    uint32_t hits = 0;
+    for (int rep = 0; rep < 300; rep++) {
+        DevList l;
+        std::vector<uint32_t> buf;              // what the buffer holds
+        std::vector<std::vector<uint32_t>> graph;
+        const bool captures = rep % 2 != 0;
+        size_t cap = 16;
+        for (int n = 0; n < 60; n++) {
+            if (captures && rng() % 4 == 0 && !graph.empty()) {
+                buf = graph[rng() % graph.size()];      // a replay
+                continue;
+            }
+            if (rng() % 16 == 0) {              // the buffer grows: its contents are gone
+                cap *= 2;
+                buf.clear();
+                graph.clear();
+            }
+            const bool captured = captures && rng() % 8 == 0;
+            const std::vector<uint32_t> what = {1u + (uint32_t)(rng() % 2), (uint32_t)(rng() % 3)};
+            if (captured) {                     // recorded, not run
+                l.take(true);
+                l.set(what, cap);
+                graph.push_back(what);
+            } else if (l.holds(what, cap)) {
+                CHECK(buf == what);
+                hits++;
+            } else {
+                l.take(false);
+                buf = what;
+                if (rng() % 4)                  // (else an upload without a kept list)
+                    l.set(what, cap);
+            }
+        }
+    }
+    CHECK(hits > 500);
+}
+
 int main()
 {
     std::mt19937 rng(20261202);
+    check_lists(rng);
     check_slots(rng);
     check_pages(rng);
     check_oracle(rng);
