@@ -64,7 +64,12 @@ hipError_t scratch_address(int dev, uint8_t **out)
 void *dev_alloc(size_t bytes)
 {
     std::lock_guard<std::mutex> lk(g_alloc_mu);
-    return g_alloc(bytes ? bytes : 1, g_alloc_user);
+    void *p = g_alloc(bytes ? bytes : 1, g_alloc_user);
+    // a refused hipMalloc stays the thread's last error, which the next
+    // launch's check would take for its own
+    if (!p)
+        (void)hipGetLastError();
+    return p;
 }
 
 void dev_free(void *p)

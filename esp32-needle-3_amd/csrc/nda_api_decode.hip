@@ -41,7 +41,7 @@ static const uint32_t *decode_order(nda_ctx *c, uint32_t rows, hipStream_t st)
     std::vector<uint32_t> ord(rows);
     for (uint32_t b = 0; b < rows; b++)
         ord[first[top - tiles[b]]++] = b;
-    if (grow_buf(c, c->d_order, c->order_cap, rows, std::max<size_t>(rows, 4096)) ||
+    if (!optional_buf(c, c->d_order, c->order_cap, rows, std::max<size_t>(rows, 4096)) ||
         upload(c, c->d_order, ord.data(), (size_t)rows * 4, st)) {
         c->order_rows = 0;
         return nullptr;

@@ -159,8 +159,8 @@ int prefill_reserve(nda_ctx *c, PrefillPlan &pl)
         return rc;
     if (int rc = ensure_pf(c, 8 * pl.n_items))
         return rc;
-    if (pl.ksplit &&
-        ensure_buf(c, c->d_pf_part, c->pf_part_cap, pl.rows * c->cfg.n_heads * pl.ksplit * PF_PART_STRIDE))
+    const size_t parts = pl.rows * c->cfg.n_heads * pl.ksplit * PF_PART_STRIDE;
+    if (pl.ksplit && !optional_buf(c, c->d_pf_part, c->pf_part_cap, parts, parts))
         pl.ksplit = 0;
     return NDA_OK;
 }

@@ -215,6 +215,20 @@ int grow_buf(nda_ctx *c, T *&buf, size_t &cap, size_t need, size_t n_alloc)
     return NDA_OK;
 }
 
+// grow_buf for a buffer that a call can do without: whether it holds `need`
+// now. A refusal leaves nothing, nda_last_error's text included.
+template <typename T>
+bool optional_buf(nda_ctx *c, T *&buf, size_t &cap, size_t need, size_t n_alloc)
+{
+    if (need <= cap)
+        return true;
+    std::string err;
+    err.swap(c->err);
+    const bool ok = grow_buf(c, buf, cap, need, n_alloc) == NDA_OK;
+    err.swap(c->err);
+    return ok;
+}
+
 int ensure_rows(nda_ctx *c, size_t rows);
 int ensure_part(nda_ctx *c, size_t floats);
 int ensure_pf(nda_ctx *c, size_t n);

@@ -35,7 +35,9 @@ FREE = C.CFUNCTYPE(None, C.c_void_p, C.c_void_p)
 
 class FailingAllocator:
     """hipMalloc / hipFree; refuses every request while `armed`, or only the
-    n-th request counted from `refuse_nth` being set."""
+    n-th request counted from `refuse_nth` being set. With `leave_error` a
+    refusal leaves an error as the thread's last one, as a refused hipMalloc
+    does (here of a host call: a device number that does not exist)."""
 
     def __init__(self):
         self.hip = C.CDLL("libamdhip64.so")
@@ -45,6 +47,7 @@ class FailingAllocator:
         self.hip.hipFree.restype = C.c_int
         self.armed = False
         self.refuse_nth = 0
+        self.leave_error = False
         self.seen = 0
         self.refused = 0
         self._alloc = ALLOC(self.alloc)
@@ -54,6 +57,8 @@ class FailingAllocator:
         self.seen += 1
         if self.armed or (self.refuse_nth and self.seen == self.refuse_nth):
             self.refused += 1
+            if self.leave_error:
+                assert self.hip.hipSetDevice(1 << 20) != 0
             return None
         p = C.c_void_p()
         return p.value if self.hip.hipMalloc(C.byref(p), nbytes) == 0 else None

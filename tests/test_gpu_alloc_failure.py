@@ -264,3 +264,41 @@ def test_two_launch_step_refused_before_its_append(allocator):
         ctx.seq_reset(b)
     ctx.prefix_free(pid)
     ctx.close()
+
+
+def test_split_prefill_without_memory_for_its_parts(allocator):
+    """A prefill of few work items splits its keys into parts of a buffer of
+    their own. With that buffer alone refused, by an allocator whose refusal
+    leaves a HIP error behind, the call runs whole: NDA_OK, the same outputs
+    to the split's tolerance, nothing allocated and nothing reported. With
+    memory the same call splits."""
+    N = nda()
+    nh, d, L, n = 8, 64, 600, 40
+    rng = np.random.default_rng(52)
+    kf, vf = (O.f32_to_f16_bits(rng.standard_normal((L, nh, d)).astype(np.float32)) for _ in range(2))
+    x = [rng.standard_normal((n, nh, d)).astype(np.float32) for _ in range(3)]
+    bufs = [N.DevBuf.from_array(a) for a in x]
+    ctx = N.Context(1, nh, nh, d, d, L + 64, kv_dtype=O.KV_F16, max_seqs=2)
+    out = N.DevBuf(n * nh * d * 4)
+    ctx.prefill(0, [n], *bufs, out, seq_ids=[1])         # short: sizes the staging, splits nothing
+    ctx.kv_write(0, 0, 0, kf, vf)
+    ctx.seq_set_pos(0, L)
+    ctx.sync()
+    got = []
+    for refuse in (True, False):
+        dev_bytes, said = ctx.device_bytes, N.lib().nda_last_error(ctx.h)
+        allocator.armed = allocator.leave_error = refuse
+        before = allocator.seen
+        ctx.prefill(0, [n], *bufs, out, seq_ids=[0])
+        allocator.armed = False
+        ctx.sync()
+        assert allocator.seen == before + 1              # the parts' buffer
+        assert (ctx.device_bytes == dev_bytes) == refuse and N.lib().nda_last_error(ctx.h) == said
+        got.append(out.to_array(np.float32, (n, nh * d)))
+        kk, vv, _, _ = ctx.kv_read(0, 0, 0, L + n)
+        for t in (0, 17, n - 1):
+            view = O.kv_view(kk, vv, None, None, nh, L + n, 0, L + t, O.KV_F16)
+            want = O.attend_view(view, x[0][t].ravel())
+            assert float(np.abs(got[-1][t] - want).max()) <= 2.5e-5, (refuse, t)
+    assert float(np.abs(got[0] - got[1]).max()) <= 2.5e-5
+    ctx.close()
