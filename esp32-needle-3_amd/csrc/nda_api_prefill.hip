@@ -159,8 +159,11 @@ int prefill_reserve(nda_ctx *c, PrefillPlan &pl)
         return rc;
     if (int rc = ensure_pf(c, 8 * pl.n_items))
         return rc;
-    const size_t parts = pl.rows * c->cfg.n_heads * pl.ksplit * PF_PART_STRIDE;
-    if (pl.ksplit && !optional_buf(c, c->d_pf_part, c->pf_part_cap, parts, parts))
+    // taken once, for the most that prefill_ksplit's rule gives (16 waves of
+    // 32 rows per CU, 36 MB): growing it would drain the device
+    const size_t parts = pl.rows * c->cfg.n_heads * pl.ksplit * PF_PART_STRIDE,
+                 most = std::max(parts, (size_t)c->cus * 16 * 32 * PF_PART_STRIDE);
+    if (pl.ksplit && !optional_buf(c, c->d_pf_part, c->pf_part_cap, parts, most))
         pl.ksplit = 0;
     return NDA_OK;
 }

@@ -301,4 +301,17 @@ def test_split_prefill_without_memory_for_its_parts(allocator):
             want = O.attend_view(view, x[0][t].ravel())
             assert float(np.abs(got[-1][t] - want).max()) <= 2.5e-5, (refuse, t)
     assert float(np.abs(got[0] - got[1]).max()) <= 2.5e-5
+    # a longer split call needs no more of it
+    ctx2 = N.Context(1, nh, nh, d, d, 4096, kv_dtype=O.KV_F16, max_seqs=2)
+    big = [N.DevBuf(512 * nh * d * 4) for _ in range(4)]
+    for i, b in enumerate(big[:3]):
+        b.fill_normal(512 * nh * d, 0, 80 + i)
+    ctx2.prefill(0, [400], *big, seq_ids=[0])           # 4 parts (the staging's first sizes hold both calls)
+    allocator.armed = True
+    refused = allocator.refused
+    ctx2.prefill(0, [512], *big, seq_ids=[0])           # 8
+    allocator.armed = False
+    ctx2.sync()
+    assert allocator.refused == refused
+    ctx2.close()
     ctx.close()
