@@ -1368,7 +1368,7 @@ void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFr
 
     float4v acc[4] = {};                        // O^T: dims 16 d + 4 g + i, column r
     float m = -FLT_MAX, lsum = 0.0f;
-    int vexp = 0;                               // several waves: acc counts in 2^(vexp - 7) (see the tile)
+    int pexp = 0;                               // several waves: acc counts in 2^(pexp - 15) (see the tile)
     const float neg1 = opaque_neg1();
 
     // the gate of this lane's output dims 16 d + 4 g + [0, 4), loaded with
@@ -1376,7 +1376,7 @@ void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFr
     // (several waves: wave d emits dims 16 d + 4 g + [0, 4))
     const float *gt = a.gate ? a.gate + qrow * DV : nullptr;
     float4 gv4[4];
-    if (NW > 1 && gt && wave < 4)
+    if (NW >= 8 && gt && wave < 4)
         gv4[0] = *reinterpret_cast<const float4 *>(gt + 16 * wave + 4 * g);
 
     // tile j: the load of the next tile (references fetched a tile ago), the
@@ -1465,6 +1465,28 @@ void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFr
                     vsc[4 * kb + i] = out ? 0.0f : vsc[4 * kb + i];
                 }
         }
+        if constexpr (NW > 1) {
+            // A position whose v is all zero is stored with scale 1, which
+            // would set the exponent below far above the others': scale 0
+            // gives the same product. (Rare: scales of 1 are looked at.)
+            bool one = false;
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                one |= vsc[i] == 1.0f;
+            if (__builtin_expect(__ballot(one) != 0, 0)) {
+                static_assert(DV == 64, "half a V row of 64 codes per lane");
+                int le = lane;          // (opaque: nothing of this is held over the tiles)
+                asm volatile("" : "+v"(le));
+                const u32x4 *vr = reinterpret_cast<const u32x4 *>(lds + KB + (le & 31) * VSTR + 32 * (le >> 5));
+                u32x4 any = vr[0];
+                any |= vr[1];
+                const uint64_t b = __ballot((any.x | any.y | any.z | any.w) != 0);
+                const uint32_t nz = ((uint32_t)b | (uint32_t)(b >> 32)) >> (8 * (le >> 4));  // from key 8 g on: has codes
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    vsc[i] = vsc[i] == 1.0f && ((nz >> i) & 1u) == 0 ? 0.0f : vsc[i];
+            }
+        }
         // the column's tile max over its 32 keys: 8 in this lane, then across
         // the four lane groups (lanes r + 16 g)
         const float y0 = max3(st[0][0], st[0][1], st[0][2]), y1 = max3(st[0][3], st[1][0], st[1][1]);
@@ -1496,29 +1518,6 @@ void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFr
                     st[kb] -= d;
             }
         }
-        if constexpr (NW > 1) {
-            // These launches took over from fp32 products, whose accuracy
-            // the fp16 pairs reach if no lo half is subnormal and hi is
-            // rounded to nearest: the v scales (about 0.02) are brought to
-            // 2^7 by a power of two that follows the largest seen, as m
-            // follows the scores.
-            float vm = max3(max3(vsc[0], vsc[1], vsc[2]), max3(vsc[3], vsc[4], vsc[5]), max3(vsc[6], vsc[7], vsc[7]));
-            vm = max3(vm, __shfl_xor(vm, 16, 64), vm);
-            vm = max3(vm, __shfl_xor(vm, 32, 64), vm);
-            const int ve = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_expf(vm));
-            if (FIRST || ve > vexp) {
-                if constexpr (!FIRST)
-#pragma unroll
-                    for (int d = 0; d < 4; d++)
-#pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            acc[d][i] = ldexpf(acc[d][i], vexp - ve);
-                vexp = ve;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                vsc[i] = ldexpf(vsc[i], 7 - vexp);      // weight * scale < 2^8 * 2^7
-        }
         float p[8];
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
@@ -1529,6 +1528,35 @@ void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFr
 #pragma unroll
         for (int i = 0; i < 8; i++)
             p[i] *= vsc[i];
+        if constexpr (NW > 1) {
+            // These launches took over from fp32 products, whose accuracy
+            // the fp16 parts reach if no lo part that counts is subnormal
+            // and hi is rounded to nearest: a column's products of weight
+            // and v scale are brought to 2^15 by a power of two that follows
+            // the largest seen, as m follows the scores (none yet: below
+            // every product, so that the first one sets it).
+            float pm = max3(max3(p[0], p[1], p[2]), max3(p[3], p[4], p[5]), max3(p[6], p[7], p[7]));
+            const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(pm), __float_as_uint(pm), false, false);
+            pm = max3(pm, __uint_as_float(s16[0]), __uint_as_float(s16[1]));
+            const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(pm), __float_as_uint(pm), false, false);
+            pm = max3(pm, __uint_as_float(s32[0]), __uint_as_float(s32[1]));
+            const int pe = max(pm > 0.0f ? __builtin_amdgcn_frexp_expf(pm) : -110, -110);
+            if constexpr (FIRST) {
+                pexp = pe;
+            } else if (__ballot(pe > pexp) != 0) {
+                const int d = min(pexp - pe, 0);
+#pragma unroll
+                for (int dd = 0; dd < 4; dd++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        acc[dd][i] = ldexpf(acc[dd][i], d);
+                pexp -= d;
+            }
+            const float f = ldexpf(1.0f, 15 - pexp);
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                p[i] *= f;
+        }
         // P^T operand (hi, lo): slots = keys 8 g .. 8 g + 7; hi = p rounded
         // toward zero (several waves: to nearest) to fp16, lo = the remainder
         u32x4 phw, plw, pxw;
@@ -1613,11 +1641,13 @@ void decode_mfma_kernel(PrefillArgs a, std::conditional_t<FRONT, FrontArgs, NoFr
         // left max -FLT_MAX and zero sums: its weight is 0.
         // (A wave's own LDS accesses complete in order.)
         __builtin_amdgcn_wave_barrier();
+        if (NW < 8 && gt)
+            gv4[0] = *reinterpret_cast<const float4 *>(gt + 16 * wave + 4 * g);
 #pragma unroll
         for (int d = 0; d < 4; d++) {
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                acc[d][i] = ldexpf(acc[d][i], vexp - 7);
+                acc[d][i] = ldexpf(acc[d][i], pexp - 15);
             *reinterpret_cast<float4v *>(lds + 16 * (64 * d + lane)) = acc[d];
         }
         *reinterpret_cast<float2 *>(lds + 4096 + 8 * lane) = float2{m, lsum};

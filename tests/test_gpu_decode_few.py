@@ -32,9 +32,10 @@ def attend(q, k, v, gate):
     return out / (1 + np.exp(-gate.astype(np.float64)))
 
 
-def check(nh, nkv, qk, f16, lens, seed, page=16, fused=True, vscale=None, tol=TOL):
+def check(nh, nkv, qk, f16, lens, seed, page=16, fused=True, vscale=None, tol=TOL, least=1.0):
     """One token of each sequence b behind lens[b] positions; nda_step, or an
-    append and a decode. vscale [rows]: per-position factors of v."""
+    append and a decode. vscale [rows]: per-position factors of v. Errors are
+    relative to a row's largest output, or to `least` where that is more."""
     N = nda()
     vd, B = 64, len(lens)
     rng = RNG(seed)
@@ -54,6 +55,8 @@ def check(nh, nkv, qk, f16, lens, seed, page=16, fused=True, vscale=None, tol=TO
     q = rng.standard_normal((B, nh, qk)).astype(np.float32)
     kn = rng.standard_normal((B, nkv, qk)).astype(np.float32)
     vn = rng.standard_normal((B, nkv, vd)).astype(np.float32)
+    if vscale is not None:
+        vn *= np.float32(vscale(total)[-1])
     gate = rng.standard_normal((B, nh, vd)).astype(np.float32)
     bufs = [N.DevBuf.from_array(a) for a in (q, kn, vn, gate)]
     out = N.DevBuf(B * nh * vd * 4)
@@ -78,7 +81,7 @@ def check(nh, nkv, qk, f16, lens, seed, page=16, fused=True, vscale=None, tol=TO
         else:
             assert np.array_equal(kr[-1], kn[b].astype(np.float16)) and np.array_equal(vr[-1], vn[b].astype(np.float16))
         want = attend(q[b], kr.astype(np.float64) * sk[..., None], vr.astype(np.float64) * sv[..., None], gate[b])
-        worst = max(worst, float(np.abs(got[b] - want).max() / max(1.0, np.abs(want).max())))
+        worst = max(worst, float(np.abs(got[b] - want).max() / max(least, np.abs(want).max())))
     ctx.close()
     print("[gpu-case] heads %d/%d qk %d %s rows %d page %d: %.3g" % (nh, nkv, qk, "f16" if f16 else "i8", B, page, worst),
           flush=True)
@@ -106,6 +109,15 @@ def test_mfma_v_scales(f):
     """v rows whose scales span many powers of two, either way, and zero rows:
     errors relative to the largest output, which the largest rows make."""
     check(12, 2, 48, False, [277], 3, vscale=f)
+
+
+@pytest.mark.parametrize("rows", [1, 130])
+def test_mfma_zero_v_before_small_v(rows):
+    """A wave's first key tile with v all zero, then v of about 1e-6: the
+    scales' running exponent starts at the first nonzero one (8 and 4 waves
+    over 32 tiles; every fourth tile is zero)."""
+    f = lambda n: np.where(np.arange(n) % 1000 // 32 % 4, 1e-6, 0.0)     # noqa: E731
+    check(12, 2, 48, False, [1000] * rows, 4, vscale=f, least=0.0)
 
 
 @pytest.mark.parametrize("nh,nkv,qk,f16", [(12, 2, 48, True), (8, 8, 64, True), (8, 8, 64, False), (6, 2, 36, False),
