@@ -35,7 +35,9 @@ void *default_alloc(size_t bytes, void *)
 }
 void default_free(void *p, void *) { (void)hipFree(p); }
 
-std::mutex g_alloc_mu;
+// held over the pair's calls (one at a time in the process); recursive, since
+// an allocator may itself give blocks back (a garbage collector that runs in it)
+std::recursive_mutex g_alloc_mu;
 nda_alloc_fn g_alloc = default_alloc;
 nda_free_fn g_free = default_free;
 void *g_alloc_user = nullptr;
@@ -63,7 +65,7 @@ hipError_t scratch_address(int dev, uint8_t **out)
 
 void *dev_alloc(size_t bytes)
 {
-    std::lock_guard<std::mutex> lk(g_alloc_mu);
+    std::lock_guard<std::recursive_mutex> lk(g_alloc_mu);
     void *p = g_alloc(bytes ? bytes : 1, g_alloc_user);
     // a refused hipMalloc stays the thread's last error, which the next
     // launch's check would take for its own
@@ -76,7 +78,7 @@ void dev_free(void *p)
 {
     if (!p)
         return;
-    std::lock_guard<std::mutex> lk(g_alloc_mu);
+    std::lock_guard<std::recursive_mutex> lk(g_alloc_mu);
     g_free(p, g_alloc_user);
 }
 
@@ -1155,7 +1157,7 @@ int nda_set_allocator(nda_alloc_fn alloc, nda_free_fn free_fn, void *user)
 {
     if (!alloc != !free_fn)
         return NDA_ERR_ARG;
-    std::lock_guard<std::mutex> lk(g_alloc_mu);
+    std::lock_guard<std::recursive_mutex> lk(g_alloc_mu);
     g_alloc = alloc ? alloc : default_alloc;
     g_free = alloc ? free_fn : default_free;
     g_alloc_user = alloc ? user : nullptr;

@@ -8,6 +8,7 @@ host; every kernel that runs still gets valid memory. After each refused call
 the test checks that positions and device bytes are as before, that the page
 pool lost nothing (it is filled to its last page afterwards), and that the
 same call then succeeds with outputs matching the oracle."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -264,6 +265,19 @@ def test_two_launch_step_refused_before_its_append(allocator):
         ctx.seq_reset(b)
     ctx.prefix_free(pid)
     ctx.close()
+
+
+def test_allocator_that_frees_blocks(allocator, monkeypatch):
+    """An allocator that gives another block back while it allocates (Python's
+    garbage collector, run inside it, does so for buffers in cycles)."""
+    N = nda()
+    old = [N.DevBuf(256) for _ in range(2)]
+    real = allocator.alloc
+    monkeypatch.setattr(allocator, "alloc", lambda n, user: (old.pop().free() if old else None, real(n, user))[1])
+    allocator._alloc = type(allocator._alloc)(allocator.alloc)
+    N._check(N.lib().nda_set_allocator(C.cast(allocator._alloc, C.c_void_p), C.cast(allocator._free, C.c_void_p), None))
+    new = N.DevBuf.from_array(np.arange(8, dtype=np.float32))
+    assert len(old) == 1 and np.array_equal(new.to_array(np.float32, (8,)), np.arange(8))
 
 
 def test_split_prefill_without_memory_for_its_parts(allocator):
