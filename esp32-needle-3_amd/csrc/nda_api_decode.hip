@@ -474,9 +474,12 @@ int nda_decode_noalloc(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t
 // engine session) fuse both into one launch: the decode work-group owning
 // the new slot quantises and stores it before attending. Large batches keep
 // two launches: a store plus barrier at the head of every one of tens of
-// thousands of work-groups costs more than the separate append kernel; GQA
-// groups the MFMA decode serves switch to it (and so to two launches) from
-// 4 work items per CU. Batches on one shared prefix that its decode pass
+// thousands of work-groups costs more than the separate append kernel. GQA
+// groups that the MFMA decode serves go there where it takes one wave per
+// row, from 5 work items per CU on (12/2 heads, rows of 213-383 positions,
+// us: 512 sequences 12.7 fused, 15.7 as two launches; 640, the last fused,
+// 17.4 and 19.4; beyond, the fused launch would be the VALU kernel's, 40).
+// Batches on one shared prefix that its decode pass
 // serves fuse the store into the own-positions pass: about the same GPU
 // time as a separate append (1024 sequences on a 213-token prefix: 53.6-56.2
 // against 54.4 us per layer step), one launch fewer to enqueue (whole steps
@@ -492,7 +495,7 @@ int nda_step(nda_ctx *c, uint32_t layer, uint32_t nseq, const uint32_t *ids, con
     if (c && layer < c->cfg.n_layers && check_ids(c, nseq, ids) == NDA_OK &&
         prefix_split_batch(c, nseq, ids, &pfx, &nsh, &mt) && prefix_split_on(nsh, mt))
         return decode_impl(c, layer, nseq, ids, q, k, v, gate, out, stream);
-    if (c && (units >= 16ull * (uint64_t)c->cus || (mfma_decode_geo(c) && units >= 4ull * (uint64_t)c->cus))) {
+    if (c && (units >= 16ull * (uint64_t)c->cus || (mfma_decode_geo(c) && mfma_decode_waves(c, nseq) == 1))) {
         // The decode's buffers first: once the append has stored this
         // position, a decode that fails for want of memory would leave the
         // step half done.
