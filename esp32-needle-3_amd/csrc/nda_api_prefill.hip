@@ -135,9 +135,10 @@ int prefill_plan(nda_ctx *c, uint32_t nseq, const uint32_t *ids, const uint32_t 
     std::vector<std::array<uint32_t, 3>> bins[8];
     size_t items = 0;
     pl.n_items = 8 * (size_t)prefill_bins(c, nseq, ids, n_tokens, pl.rep, pl.trows, bins, &items);
-    // fp16 K/V only: an int8 prefill's weights carry the v scales, and its
-    // errors on keys with large scores (3e-5 against 64 bits, where fp16's are
-    // 1e-6) follow the order of the tiles
+    // fp16 K/V only: on keys with 8-sigma logits an int8 prefill is about 3e-5
+    // from 64 bits in either form (fp16 1e-6 or less), and the two forms came
+    // out 3.4e-5 apart, so an int8 prompt's results would follow how many work
+    // items share its launch
     if (!pl.valu && c->geo.kv_f16)
         pl.ksplit = prefill_ksplit(c, items, pl.tab_cap, pl.waves);
     c->plan = pl;

@@ -503,17 +503,17 @@ void prefill_kernel(PrefillArgs a)
     // rows are decode queries of sequences attached to it, packed across
     // them, and it leaves each row's softmax state for the sequences' own
     // positions to continue.
-    // Split keys (a.ksplit parts, blockIdx.y): the work-group attends its
-    // share of the item's tiles and leaves the rows' states for
+    // Split keys (a.ksplit parts, blockIdx.y; fp16 K/V only): the work-group
+    // attends its share of the item's tiles and leaves the rows' states for
     // pf_merge_kernel.
-    const bool partial = a.part != nullptr && a.ksplit == 0;
+    const bool partial = a.part != nullptr && (ES != 2 || a.ksplit == 0);
     io.own_len = partial ? 0 : kmax - n_sh;         // own slots [0, own_len) are touched
     io.nfs = n_sh / PF_KT;
     io.psh = n_sh % PF_KT != 0;
     io.jfull = io.nfs + (partial ? 0 : (kfull - n_sh) / PF_KT);   // + own tiles visible to every row
     io.ntile = io.nfs + io.psh + (io.own_len + PF_KT - 1) / PF_KT;
     io.t0 = 0;
-    if (a.ksplit) {
+    if (ES == 2 && a.ksplit) {
         const int all = io.ntile, y = (int)blockIdx.y, S = (int)a.ksplit;
         io.t0 = (int)((int64_t)all * y / S);
         io.ntile = (int)((int64_t)all * (y + 1) / S) - io.t0;
