@@ -224,6 +224,67 @@ def test_front_multi_token_large_launch(shape, kv_dtype):
             assert np.array_equal(bits(ctx.front_hist(b)), bits(want)), (rnd, b)
 
 
+@pytest.mark.parametrize("shape,rows,page,taps", [
+    ((12, 2, 48, 64), 128, 16, 3), ((12, 2, 48, 64), 129, 16, 3), ((12, 2, 48, 64), 300, 32, 5),
+    ((12, 2, 48, 64), 640, 16, 3), ((12, 2, 48, 64), 641, 16, 3), ((12, 2, 48, 64), 40, 64, 6),
+    ((8, 2, 64, 64), 200, 64, 3), ((16, 2, 64, 64), 300, 16, 2), ((6, 1, 64, 64), 257, 32, 3),
+])
+def test_attention_equals_front_store_decode(shape, rows, page, taps):
+    """nda_attention of int8 GQA batches, whose decode launch runs the front
+    and the store itself (eight waves per (row, kv-head) up to one item per
+    CU, four up to five, separate launches beyond), against nda_front +
+    nda_kv_append + nda_decode: outputs, stored codes and tap histories bit
+    for bit. Sequences of 0 to 1000 positions, a third of them on a shared
+    prefix, a third past the window; two steps, of all and of listed ids."""
+    N = nda()
+    nh, nkv, qk, vd = shape
+    say("attention against its parts", shape, rows, page, taps)
+    W, npre, L = 1000, 70, 2
+    rng = np.random.default_rng(rows + page)
+    fw = make_weights(rng, L, nh, nkv, qk, vd, taps)
+    lens = [(0, 1, 40, 200, 333, 500, 640, 929)[b % 8] for b in range(rows)]
+    ctxs = []
+    for _ in range(2):
+        r2 = np.random.default_rng(rows)
+        c = N.Context(L, nh, nkv, qk, vd, W, kv_dtype=O.KV_INT8, max_seqs=rows + 1, page_size=page)
+        c.front_init(taps, 10000.0)
+        for li in range(L):
+            c.front_weights(li, *fw.arrays(li))
+        c.seq_set_pos(rows, npre)
+        c.kv_fill_normal(1, seed=5, seq_ids=[rows])
+        pid = c.prefix_build(rows)
+        for b in range(rows):
+            if b % 3 == 0:
+                c.seq_attach(b, pid)
+            c.seq_set_pos(b, lens[b] + (npre if b % 3 == 0 else W if b % 3 == 1 else 0))
+        c.kv_fill_normal(rows, seed=int(r2.integers(1000)))
+        ctxs.append(c)
+    dims = (nh * qk, nkv * qk, nkv * vd, nh * vd)
+    for step in range(2):
+        ids = None if step == 0 else [int(x) for x in rng.permutation(rows)]
+        for li in range(L):
+            bufs = [N.DevBuf.from_array(rng.standard_normal((rows, d)).astype(np.float32)) for d in dims]
+            outs = [N.DevBuf(rows * nh * vd * 4) for _ in range(2)]
+            ctxs[0].attention(li, rows, *bufs[:3], outs[0], gate=bufs[3], seq_ids=ids)
+            f = [N.DevBuf(rows * d * 4) for d in dims[:3]]
+            ctxs[1].front(li, rows, *bufs[:3], *f, seq_ids=ids)
+            ctxs[1].kv_append(li, rows, f[1], f[2], seq_ids=ids)
+            ctxs[1].decode(li, rows, f[0], outs[1], gate=bufs[3], seq_ids=ids)
+            got = [o.to_array(np.uint32, (rows, nh * vd)) for o in outs]
+            assert np.isfinite(got[0].view(np.float32)).all()
+            assert np.array_equal(*got), (step, li, int((got[0] != got[1]).any(1).sum()))
+            for b in range(0, rows, 7):
+                p = ctxs[0].seq_state(b)[0]
+                for x, y in zip(*(c.kv_read(li, b, p, 1) for c in ctxs)):
+                    assert np.array_equal(x, y), (step, li, b)
+        for c in ctxs:
+            c.advance(rows)
+    for b in range(0, rows, 5):
+        assert np.array_equal(*(bits(c.front_hist(b)) for c in ctxs)), b
+    for c in ctxs:
+        c.close()
+
+
 @pytest.mark.parametrize("shape,kv_dtype", [((8, 2, 64, 64), O.KV_INT8), ((8, 2, 64, 64), O.KV_F16),
                                              ((10, 2, 36, 20), O.KV_INT8), ((7, 1, 64, 64), O.KV_F16)])
 def test_attention_batched_sessions(shape, kv_dtype):

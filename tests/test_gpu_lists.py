@@ -73,3 +73,94 @@ def test_prefill_lists(between):
             one.advance(len([i for i, m in zip(ids, lens) if m]), [i for i, m in zip(ids, lens) if m], 1)
             done.append(([i for i, m in zip(ids, lens) if m], 1))
     one.close()
+
+
+def ops(rng, groups):
+    """A call of each kind on other sequences, lengths and positions than the
+    last of its kind, or on the same again."""
+    kept = {}
+    for _ in range(60):
+        kind = rng.choice(["front", "prefill", "step", "step", "advance"])
+        if kind in kept and rng.random() < 0.4:
+            yield kept[kind]
+            continue
+        if kind == "step":
+            g = groups[rng.integers(len(groups))]
+            what = (kind, [int(x) for x in (g if rng.random() < 0.5 else rng.permutation(g))], None)
+        else:
+            ids = [int(x) for x in rng.permutation(groups[rng.integers(len(groups))])[:rng.integers(1, 5)]]
+            if kind == "front" and rng.random() < 0.3:
+                what = (kind, ids, None)
+            else:
+                what = (kind, ids, [int(x) for x in rng.integers(0 if len(ids) > 1 else 1, 4, len(ids))])
+                what[2][0] = max(1, what[2][0])
+        kept[kind] = what
+        yield what
+
+
+@pytest.mark.parametrize("streams", [1, 2])
+def test_lists_of_every_kind(streams):
+    """Fronts, prefills and decode steps over two shared prefixes of different
+    lengths (128 sequences each, which take the shared-prefix pass) in any
+    order, each over two layers, from one stream or two in turn: outputs and
+    histories equal those of a context whose every call is preceded by one of
+    each kind on a spare sequence, so that no list of it is ever held."""
+    N = nda()
+    taps, spare, per = 3, 256, 128
+    rng = np.random.default_rng(5)
+    w = [(rng.standard_normal((taps, NH * d)) * 0.5).astype(np.float32) for d in (QK, QK, VD)]
+    norms = [(rng.standard_normal(QK) * 0.25).astype(np.float32) for _ in range(2)]
+    ctxs = []
+    for _ in range(2):
+        c = N.Context(LAYERS, NH, NH, QK, VD, W, kv_dtype=N.KV_F16, max_seqs=spare + 1)
+        c.front_init(taps, 10000.0)
+        for li in range(LAYERS):
+            c.front_weights(li, *w, *norms)
+        for g, npre in enumerate((64, 110)):
+            c.seq_set_pos(g * per, npre)
+            c.kv_fill_normal(1, seed=g, seq_ids=[g * per])
+            pid = c.prefix_build(g * per)
+            for b in range(g * per, (g + 1) * per):
+                c.seq_attach(b, pid)
+        ctxs.append(c)
+    st = [N.vp() for _ in range(streams)]
+    if streams > 1:
+        for s in st:
+            N._check(N.lib().nda_stream_create(N.C.byref(s)))
+    one = [N.DevBuf.from_array(a) for a in data(1, 1)]
+    dump = [N.DevBuf(NH * VD * 4) for _ in range(3)]
+    for n, (kind, ids, m) in enumerate(ops(rng, [range(per), range(per, 2 * per)])):
+        if kind == "advance":
+            for c in ctxs:
+                c.advance(len(ids), ids, 1, stream=st[n % streams])
+            continue
+        rows = len(ids) if m is None else sum(m)
+        for layer in range(LAYERS):
+            x = [N.DevBuf.from_array(a) for a in data(100 * n + layer, rows)]
+            got = []
+            for c in ctxs:
+                s = st[n % streams] if c is ctxs[0] else None
+                if c is ctxs[1]:
+                    c.front(layer, 1, *one, *dump, seq_ids=[spare])
+                    c.prefill(layer, [1], *one, dump[0], seq_ids=[spare])
+                y = [N.DevBuf(rows * NH * d * 4) for d in (QK, QK, VD)]
+                if kind == "front":
+                    c.front(layer, len(ids), *x, *y, n_tokens=m, seq_ids=ids, stream=s)
+                elif kind == "prefill":
+                    c.prefill(layer, np.asarray(m, np.uint32), *x, y[0], seq_ids=ids, stream=s)
+                else:
+                    c.step(layer, len(ids), *x, y[0], seq_ids=ids, stream=s)
+                got.append(y)
+            for c in ctxs:
+                c.sync()
+            N.device_sync()
+            for a, b in list(zip(*got))[:3 if kind == "front" else 1]:
+                a, b = (t.to_array(np.uint32, (rows, NH * QK)) for t in (a, b))
+                assert np.array_equal(a, b), (n, kind, layer)
+    for b in range(0, 2 * per, 9):
+        assert np.array_equal(*(c.front_hist(b).view(np.uint32) for c in ctxs)), b
+    for c in ctxs:
+        c.close()
+    if streams > 1:
+        for s in st:
+            N._check(N.lib().nda_stream_destroy(s))

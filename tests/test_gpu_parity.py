@@ -655,9 +655,12 @@ def test_decode_4096_ragged_sequences_one_layer_sampled():
 
 # ------------------------------------------------------- MFMA prefill kernel
 
-def _prefill_case(kv_dtype, nh, nkv, qk, hist, ntok, seed, flags=0, outlier_p=0.0, gated=True):
+def _prefill_case(kv_dtype, nh, nkv, qk, hist, ntok, seed, flags=0, outlier_p=0.0, gated=True, split=None):
     """Sequences with `hist[b]` stored positions prefill `ntok[b]` tokens in one
-    call; every token's output against the oracle over positions [0, pos+t]."""
+    call; every token's output against the oracle over positions [0, pos+t].
+    split: whether the call splits its items' key tiles over work-groups (a
+    context's first split call takes the parts' buffer, 16 waves of 32 rows x
+    68 floats per CU)."""
     N = nda()
     vd = 64
     rng = np.random.default_rng(seed)
@@ -689,9 +692,12 @@ def _prefill_case(kv_dtype, nh, nkv, qk, hist, ntok, seed, flags=0, outlier_p=0.
     v = rng.standard_normal((T, nkv, vd)).astype(np.float32)
     g = rng.standard_normal((T, nh, vd)).astype(np.float32) if gated else None
     dout = N.DevBuf(max(1, T) * nh * vd * 4)
+    dev_bytes = ctx.device_bytes
     ctx.prefill(0, ntok, N.DevBuf.from_array(q), N.DevBuf.from_array(k), N.DevBuf.from_array(v), dout,
                 gate=None if g is None else N.DevBuf.from_array(g))
     ctx.sync()
+    if split is not None:
+        assert (ctx.device_bytes - dev_bytes >= N.device_info()[1] * 16 * 32 * 68 * 4) == split
     got = dout.to_array(np.float32, (T, nh * vd))
     worst, r = 0.0, 0
     for b in range(B):
@@ -751,9 +757,11 @@ def test_prefill_small_groups_direct_and_staged_tiles(hist, ntok):
     table fits the LDS their residency leaves (224 tiles at 2 waves), and
     stage them through registers without a table otherwise: 6000 + 20
     positions (189 tiles, direct), 8000 + 40 (252 tiles, staged), 8000 + 100
-    at 4 waves (direct), with 8-sigma keys."""
+    at 4 waves (direct), with 8-sigma keys. 128 sequences of one token beside
+    them make the launch too large for its keys to be split."""
     say("prefill small groups", hist, ntok)
-    worst, _ = _prefill_case(O.KV_F16, 8, 8, 64, hist, ntok, seed=31 + ntok[0], outlier_p=1e-3)
+    worst, _ = _prefill_case(O.KV_F16, 8, 8, 64, hist + [0] * 128, ntok + [1] * 128, seed=31 + ntok[0], outlier_p=1e-3,
+                             split=False)
     assert worst <= TOL, worst
 
 
@@ -763,18 +771,28 @@ def test_prefill_small_groups_direct_and_staged_tiles(hist, ntok):
 SPLIT_TOL = 2.5e-5
 
 
-@pytest.mark.parametrize("kv_dtype,nh,nkv,qk,hist,ntok,gated", [
-    (O.KV_F16, 8, 8, 64, [2500], [40], True),                        # 64-row groups, 32 parts
-    (O.KV_F16, 8, 8, 64, [0, 700, 3, 40], [1, 300, 2, 33], False),   # empty parts, parts above the diagonal
-    (O.KV_INT8, 12, 2, 48, [600, 0], [60, 129], True),               # GQA rows, a chunk's own tiles split
-    (O.KV_INT8, 8, 8, 64, [352], [1], True),                         # the smallest: 12 tiles, one row
+@pytest.mark.parametrize("nh,nkv,qk,hist,ntok,gated,split", [
+    (8, 8, 64, [2500], [40], True, True),                        # 80 tiles in 16 parts, 64-row groups
+    (8, 8, 64, [0, 700, 3, 40], [1, 300, 2, 33], False, True),   # empty parts, parts above the diagonal
+    (12, 2, 48, [600, 0], [60, 129], True, True),                # GQA rows, staged tiles, a chunk's own tiles split
+    (8, 2, 64, [500], [33], False, True),                        # GQA rows, tiles straight into LDS
+    (8, 8, 64, [352], [1], True, True),                          # the smallest: 12 tiles, one row
+    (8, 8, 64, [320], [1], True, False),                         # 11 tiles
+    (8, 8, 64, [8300], [40], True, True),                        # 261 tiles in 32 parts, merged in two rounds
+    (8, 8, 64, [16500], [33], True, True),                       # 517 tiles in 64 parts, in four
 ])
-def test_prefill_split_keys(kv_dtype, nh, nkv, qk, hist, ntok, gated):
+def test_prefill_split_keys(nh, nkv, qk, hist, ntok, gated, split):
     """Launches of few work items split each item's key tiles over several
     work-groups and merge their states."""
-    say("prefill split keys", kv_dtype, nh, nkv, qk, hist, ntok)
-    worst, _ = _prefill_case(kv_dtype, nh, nkv, qk, hist, ntok, seed=61 + nh, gated=gated)
+    say("prefill split keys", nh, nkv, qk, hist, ntok)
+    worst, _ = _prefill_case(O.KV_F16, nh, nkv, qk, hist, ntok, seed=61 + nh, gated=gated, split=split)
     assert worst <= SPLIT_TOL, worst
+
+
+def test_prefill_int8_is_not_split():
+    say("prefill int8 whole")
+    worst, _ = _prefill_case(O.KV_INT8, 12, 2, 48, [600, 0], [60, 129], seed=73, split=False)
+    assert worst <= TOL, worst
 
 
 @pytest.mark.parametrize("npre,suffix", [(500, [40, 1]), (512, [33]), (395, [64, 3, 20])])
