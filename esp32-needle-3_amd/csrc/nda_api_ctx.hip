@@ -463,13 +463,13 @@ bool mfma_decode(const nda_ctx *c, const AttnArgs &a)
 
 // Waves per (row, kv-head) of the MFMA decode. Where one wave per item
 // leaves the chip idle, a row's tiles are split over several (12/2 heads,
-// rows of 213-383 positions, us): one session 23.9 (the VALU kernel) -> 5.2
-// with 8 waves; 600 items 15.0 with one wave, 9.8 with 4, 13.8 with 8; 1024
-// items 14.1, 10.6, 14.0; 1400 items 15.5, 14.6, 19.4; 2048 items 16.9,
-// 18.6, 26.2. Up to one item per CU 8 waves gain on long rows (16 items of
-// 700-1000 positions 8.6 against 10.6) and lose nothing on short ones.
-// Launches of several waves also fuse a step's store (the one-wave VALU
-// kernel took 40 us for it).
+// rows of 213-383 positions, us with 1, 4 and 8 waves): one session 7.8, 5.4,
+// 5.5 (the VALU kernel 23.9); 600 items 12.7, 9.0, 17.0; 1024 items 13.8,
+// 11.4, 22.3; 1280 items 15.0, 15.0, 27.4; 1400 items 15.0, 16.0, 31.1; 2048
+// items 16.5, 20.1, 42.5. Up to one item per CU 8 waves gain on long rows (16
+// items of 700-1000 positions 9.2 against 10.9) and lose 0.4 at most on
+// shorter ones. Launches of several waves also fuse a step's store (the
+// one-wave VALU kernel took 40 us for it).
 int mfma_decode_waves(const nda_ctx *c, uint32_t rows)
 {
     const uint64_t items = (uint64_t)rows * c->cfg.n_kv_heads, cus = (uint64_t)c->cus;

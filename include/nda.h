@@ -417,7 +417,12 @@ int nda_device_info(char *name, size_t name_len, int *cu_count);
 
 /* ---- kernel timing (the engine's ND_PROFILE phases, nd_model.h:238-269) ----
  * When enabled, every launch is bracketed by HIP events on its own stream and
- * the elapsed device time is accumulated per kernel kind. */
+ * the elapsed device time is accumulated per kernel kind. A launch that does
+ * the work of several kinds counts once, under the last: the store that
+ * nda_step fuses, and the front and store of nda_attention on int8 GQA
+ * batches of up to five (row, kv-head) items per CU, are part of
+ * NDA_K_DECODE (NDA_K_FRONT then counts nothing); the merge of a split-key
+ * prefill is part of NDA_K_PREFILL. */
 #define NDA_K_APPEND  0   /* ND_P_KVST */
 #define NDA_K_DECODE  1   /* ND_P_ATTN */
 #define NDA_K_COMBINE 2   /* split-KV merge */
