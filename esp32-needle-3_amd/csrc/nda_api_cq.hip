@@ -192,6 +192,8 @@ static int cq_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const flo
     a.bits = t0->bits;
     a.rowbytes = t0->rowbytes;
     a.nt = n;
+    a.waves = cq_lut_waves(t0->in_pad, t0->group, t0->ngroup, rows);
+    const uint32_t ot = a.waves ? CQ_LUT_OT : CQ_LUT_WIDE_OT;
     uint32_t tiles = 0;
     for (uint32_t i = 0; i < n; i++) {
         const nda_cq *t = ts[i];
@@ -207,7 +209,7 @@ static int cq_lut2(const nda_cq *const *ts, uint32_t n, uint32_t rows, const flo
         a.cb[i] = t->cb;
         a.out[i] = t->out;
         a.tile0[i] = tiles;
-        tiles += (t->out + CQ_LUT_OT - 1) / CQ_LUT_OT;
+        tiles += (t->out + ot - 1) / ot;
     }
     a.tile0[n] = tiles;
     return launch_cq_lut2(a, raw, (hipStream_t)stream) == hipSuccess ? NDA_OK : NDA_ERR_HIP;

@@ -1174,6 +1174,8 @@ void cq_gemm_raw_kernel(CqSplitArgs a)
 // group's words and leaves norm * sum in LDS, and the first wave adds the
 // groups up in order. The chain is a sixth as long, and 1568 outputs are 25
 // work-groups a row instead of 8.
+// WIDE: 256 outputs of one row, the groups in turn, each group's table shared
+// by the four waves (cq_lut_waves says where).
 // G: the group at compile time, 0: at run time. PREP (group 128): xh holds
 // the raw activations and each wave transforms its own group in registers,
 // lane l columns 2l and 2l + 1, the engine's butterflies stage by stage as in
@@ -1182,16 +1184,18 @@ void cq_gemm_raw_kernel(CqSplitArgs a)
 // Per launch at 768 inputs, group 128 (q/k/v/gate, 1568 outputs): 4.9 us for
 // 1 row and 7.0 us for 24, where a work-group of 256 outputs with a whole
 // chain per thread took 21.1 and 21.6 us, after a prepare launch of 4.1-4.8.
-template <int G, bool PREP>
-__global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmArgs a)
+template <int G, bool PREP, bool WIDE = false>
+__global__ __launch_bounds__(WIDE ? CQ_LUT_WIDE_OT : 64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmArgs a)
 {
 #pragma clang fp contract(off)
+    static_assert(!(WIDE && PREP), "a wave per group prepares it");
     extern __shared__ __attribute__((aligned(16))) float lut[];   // [waves][group / 2][16], then [ngroup][64]
     const int lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const uint32_t wave = WIDE ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = WIDE ? 1u : blockDim.x >> 6;
     const uint32_t group = G ? G : a.group, gw = group / 16;      // words per group
     const uint32_t tile = blockIdx.x, row = blockIdx.y, t = tensor_of(a.tile0, a.nt, tile);
-    const uint32_t o = (tile - a.tile0[t]) * CQ_LUT_OT + lane, oc = min(o, a.out[t] - 1);
+    const uint32_t o = WIDE ? (tile - a.tile0[t]) * CQ_LUT_WIDE_OT + threadIdx.x : (tile - a.tile0[t]) * CQ_LUT_OT + lane;
+    const uint32_t oc = min(o, a.out[t] - 1);
     const uint32_t *qw = reinterpret_cast<const uint32_t *>(a.packed[t] + (uint64_t)oc * a.rowbytes);
     const uint16_t *nrm = a.norms[t] + (uint64_t)oc * a.ngroup;
     const float cb[4] = {a.cb[t][0], a.cb[t][1], a.cb[t][2], a.cb[t][3]};
@@ -1211,7 +1215,7 @@ __global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmAr
                 w[4 * j + 2] = v.z;
                 w[4 * j + 3] = v.w;
             }
-        for (uint32_t p = lane; p < group / 2; p += 64) {
+        for (uint32_t p = WIDE ? threadIdx.x : lane; p < group / 2; p += WIDE ? CQ_LUT_WIDE_OT : 64) {
             float x0, x1;
             if constexpr (PREP) {
                 const uint32_t c = gi * G + 2 * p;
@@ -1254,7 +1258,10 @@ __global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmAr
                     float4{l[0] + h[i], l[1] + h[i], l[2] + h[i], l[3] + h[i]};
         }
         // a wave's LDS operations complete in order: its own table needs no barrier
-        __builtin_amdgcn_wave_barrier();
+        if constexpr (WIDE)
+            __syncthreads();
+        else
+            __builtin_amdgcn_wave_barrier();
         const float *T = T0;
         float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
         auto word = [&](uint32_t v) __attribute__((always_inline)) {
@@ -1281,7 +1288,10 @@ __global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmAr
             part[gi * 64 + lane] = r;
         else
             acc = acc + r;
-        __builtin_amdgcn_wave_barrier();
+        if constexpr (WIDE)
+            __syncthreads();
+        else
+            __builtin_amdgcn_wave_barrier();
     }
     if (nw > 1) {
         __syncthreads();
@@ -1294,17 +1304,36 @@ __global__ __launch_bounds__(64 * CQ_LUT_MAX_WAVES) void cq_lut2_kernel(CqGemmAr
         a.y[t][(uint64_t)row * a.out[t] + o] = acc;
 }
 
+// One wave per group as far as 64 KiB of LDS hold their tables and the groups'
+// sums. From 128 rows on, where launches fill the chip, a wave takes 64 columns
+// at least (512 columns in groups of 32 x 1000 outputs x 1024 rows: 96 us,
+// with 16 waves 105). Where that leaves one wave (but for groups of 128, whose
+// own instance is faster), and for groups of 512 and more, 256 outputs share a
+// table instead, the groups in turn. us, a wave per group -> 256 outputs: 2048
+// columns in one group x 512 outputs, 1 row 27.4 -> 26.4, 1024 rows 493 ->
+// 144; in groups of 512, 1 row 15.4 -> 27.3 (so not below 128 rows unless one
+// wave is left), 128 rows 33.0 -> 30.0, 1024 rows 202 -> 132.
+uint32_t cq_lut_waves(uint32_t in_pad, uint32_t group, uint32_t ngroup, uint32_t rows)
+{
+    const uint32_t tab = group * 8 * sizeof(float), sums = ngroup * 64 * sizeof(float);
+    uint32_t nw = std::min({ngroup, (uint32_t)CQ_LUT_MAX_WAVES, (65536u - sums) / tab});
+    if (rows >= 128)
+        nw = std::min(nw, in_pad / 64);
+    const bool one = nw <= 1, big = group >= 512;
+    return group != 128 && (rows >= 128 ? one || big : one && big) ? 0 : std::max(1u, nw);
+}
+
 hipError_t launch_cq_lut2(const CqGemmArgs &a, bool prep, hipStream_t s)
 {
     if (a.rows == 0 || a.nt == 0 || a.tile0[a.nt] == 0)
         return hipSuccess;
     if (a.bits != 2 || a.group % 16 || a.in_pad > CQ_LUT_MAX_IN || a.rows > 65535 || (prep && a.group != 128))
         return hipErrorInvalidValue;
-    // one wave per group as far as 64 KiB of LDS hold their tables (and,
-    // with several waves, the groups' sums); a single wave keeps its sum in
-    // a register
-    const uint32_t tab = a.group * 8 * sizeof(float), sums = a.ngroup * 64 * sizeof(float);
-    const uint32_t nw = std::max(1u, std::min({a.ngroup, (uint32_t)CQ_LUT_MAX_WAVES, (65536u - sums) / tab}));
+    const uint32_t tab = a.group * 8 * sizeof(float), sums = a.ngroup * 64 * sizeof(float), nw = a.waves;
+    if (nw == 0) {
+        hipLaunchKernelGGL((cq_lut2_kernel<0, false, true>), dim3(a.tile0[a.nt], a.rows), dim3(CQ_LUT_WIDE_OT), tab, s, a);
+        return hipGetLastError();
+    }
     const size_t lds = (size_t)nw * tab + (nw > 1 ? sums : 0);
     const dim3 grid(a.tile0[a.nt], a.rows), wg(64 * nw);
     if (prep)

@@ -189,6 +189,7 @@ struct CqPrepArgs {
  * outputs per tile in the GEMM, CQ_LUT_OT in the engine-order kernel). */
 constexpr int CQ_MAX_T = 8;
 constexpr int CQ_LUT_OT = 64;         /* engine-order kernel: outputs per work-group */
+constexpr int CQ_LUT_WIDE_OT = 256;   /*   and where they share one table */
 constexpr int CQ_LUT_MAX_WAVES = 16;  /*   and its waves at most, each on groups of its own */
 constexpr int CQ_LUT_MAX_IN = 2048;   /* its pair table, in_pad * 32 bytes of LDS, within 64 KiB */
 struct CqGemmArgs {
@@ -204,6 +205,7 @@ struct CqGemmArgs {
     uint32_t rows, in_pad, group, ngroup, bits, rowbytes;
     uint32_t in;                        /* raw activations: their width, and 1 / sqrt(group) */
     float scale;
+    uint32_t waves;                     /* engine-order kernel: cq_lut_waves */
 };
 
 /* The split-precision form of a prepared activation: xh * 2^rexp[r] as an
@@ -256,7 +258,9 @@ constexpr uint32_t CQ_RAW_MAX_G = 8;    /* cq_gemm_raw_kernel: groups (of 128 co
 
 hipError_t launch_cq_prepare(const CqPrepArgs &a, hipStream_t s);
 hipError_t launch_cq_gemm(const CqGemmArgs &a, hipStream_t s);
-/* prep: a.xh holds the raw activations (group 128 only) */
+/* Waves per 64 outputs of a row, 0: tiles of CQ_LUT_WIDE_OT outputs. */
+uint32_t cq_lut_waves(uint32_t in_pad, uint32_t group, uint32_t ngroup, uint32_t rows);
+/* prep: a.xh holds the raw activations (group 128, a.waves not 0) */
 hipError_t launch_cq_lut2(const CqGemmArgs &a, bool prep, hipStream_t s);
 hipError_t launch_cq_prepare_split(const CqPrepSplitArgs &a, hipStream_t s);
 hipError_t launch_cq_gemm_split(const CqSplitArgs &a, hipStream_t s);

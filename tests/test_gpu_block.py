@@ -157,7 +157,7 @@ def test_block_batched(shape, kv_dtype):
             c.close()
 
 
-@pytest.mark.parametrize("dm,group,rows", [(768, 128, 64), (333, 128, 1), (130, 128, 7), (2047, 128, 3), (256, 64, 5)])
+@pytest.mark.parametrize("dm,group,rows", [(768, 128, 64), (333, 128, 1), (130, 128, 7), (100, 128, 5), (2047, 128, 3), (256, 64, 5)])
 def test_block_projections_equal_the_separate_calls(dm, group, rows):
     """The block's projections of a few rows (at group 128 one launch from
     the raw activations, odd and padded widths included) equal
@@ -198,8 +198,8 @@ def test_block_projections_equal_the_separate_calls(dm, group, rows):
         t.close()
 
 
-@pytest.mark.parametrize("dm,rows", [(768, 65), (768, 96), (768, 97), (768, 512), (768, 513), (768, 608), (768, 609), (128, 70), (1024, 127),
-                                     (1152, 100), (840, 90)])
+@pytest.mark.parametrize("dm,rows", [(768, 65), (768, 96), (768, 97), (768, 512), (768, 513), (768, 608), (768, 609),
+                                     (128, 70), (1024, 127), (1152, 100), (840, 90)])
 def test_block_projections_of_many_rows(dm, rows):
     """From 65 rows on, three decode steps of the block equal the separate
     calls (nda_cq_prepare_split, nda_cq_gemm_split*, nda_step) bit for bit."""

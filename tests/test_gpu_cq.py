@@ -138,6 +138,10 @@ def test_cq_golden_reference_outputs():
     ([300, 17], 2048, 256, 4),                # the largest table (in_pad 2048)
     ([33], 100, 16, 9),                       # group 16, padded
     ([70, 70], 96, 32, 1),
+    ([300, 17], 2048, 2048, 3), ([256, 1], 500, 512, 2),     # one table of 512 and more: 256 outputs share it
+    ([70], 1024, 512, 127), ([257, 255], 1024, 512, 128),    # and from 128 rows on
+    ([257], 32, 32, 127), ([257], 32, 32, 128),              # one small group
+    ([65], 128, 128, 128), ([260], 512, 32, 128),            # one group of 128; two groups a wave
 ])
 def test_cq_lut2_bit_exact(shapes, inp, group, rows):
     """nda_cq_gemv_lut2: every output bit-identical to the engine's
