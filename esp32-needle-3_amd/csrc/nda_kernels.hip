@@ -891,13 +891,19 @@ constexpr uint32_t ATT_LONG_ITEM = 448;
 
 // Launches of few work items are bound by one work-group's walk along its
 // positions, whatever the geometry, so those of long enough rows run eight
-// waves (us, before -> now):
-//   - rep >= 4 (one wave elsewhere), up to 3 items per CU of 128 positions or
-//     more: 12/2 heads fp16, 213-383 positions, 1 sequence 24 -> 15, 32 36.5
-//     -> 17.8, 256 55 -> 28, 400 58 -> 46 (at 90 positions 240 sequences
-//     19.7 -> 21.8); in chunks of 1024 of 4-8K positions, 2 sequences fp16 90
-//     -> 26, int8 62 -> 30, 32 sequences 136 -> 43 and 85 -> 66;
-//   - rep <= 2 (two waves elsewhere), up to 2 items per CU: 8 heads, 213-383
+// waves. us, before -> now:
+//   - rep >= 4 (one wave elsewhere), up to one item per CU from 128 positions
+//     on: 12/2 heads fp16, 213-383 positions, 1 sequence 24 -> 15, 32 36.5 ->
+//     17.8 (at 90 positions 256 items 19.7 -> 21.8); in chunks of 1024 of 4-8K
+//     positions, 2 sequences fp16 90 -> 26, int8 62 -> 30;
+//   - rep >= 4, up to three items per CU: an item's merge and waves weigh more
+//     the more heads it has. Time of eight waves over one's, rep 4, 5, 6, 7 and
+//     8, fp16: 512 items at 130 positions 0.76, 0.89, 0.92, 1.26, 1.43, at 200
+//     0.58, 0.72, 0.71, 1.03, 1.12, at 300 0.42, 0.52, 0.50, 0.79, 0.79; 768
+//     items at 200 0.81, 1.00, 0.97, 1.37, 1.53, at 300 0.60, 0.74, 0.70, 1.07,
+//     1.08, at 800 0.46, 0.58, 0.49, 0.78, 0.72. int8 chunks of 750 positions:
+//     rep 6 at qk 64, 512 items 0.83, 768 1.11; rep 8, 256 items 0.65, 512 1.10;
+//   - rep <= 3 (two waves elsewhere), up to 2 items per CU: 8 heads, 213-383
 //     positions, 64 sequences fp16 22 -> 12, int8 14.7 -> 11.6 (96 sequences
 //     int8 16.8 -> 19.0); at 180 positions 60 sequences fp16 13.5 -> 9.3, but
 //     4 sequences int8 7.3 -> 8.0: the merge of eight states costs about 1 us.
@@ -905,10 +911,15 @@ constexpr int ATT_FEW_NW = 8;
 template <int ES, int REP>
 static bool att_few(const AttnArgs &a)
 {
-    const uint64_t items = (uint64_t)a.rows * a.pg.nkv * (a.max_chunks - a.chunk_lo);
+    const uint64_t items = (uint64_t)a.rows * a.pg.nkv * (a.max_chunks - a.chunk_lo), cus = a.cus;
     const uint32_t len = a.avg_len < a.chunk ? a.avg_len : a.chunk;
-    return a.chunk_lo == 0 && items <= (REP >= 4 ? 3ull : 2ull) * a.cus &&
-           len >= (REP >= 4 ? 128u : ES == 2 ? 160u : 256u);
+    if (a.chunk_lo != 0)
+        return false;
+    if (REP < 4)
+        return items <= 2 * cus && len >= (ES == 2 ? 160u : 256u);
+    if (items > (ES == 2 ? 3 : REP == 8 ? 1 : REP >= 6 ? 2 : 3) * cus)
+        return false;
+    return len >= (items <= cus ? 128u : items <= 2 * cus ? 32u * REP : (REP >= 7 ? 64u : 48u) * REP);
 }
 
 // Positions per lane group per step. fp16 at rep <= 2: 4 (80 registers, 6
