@@ -25,13 +25,15 @@
  *     calls (nda_kv_read / nda_kv_write) run on the null stream the same way.
  *     Contexts do not order each other;
  *   - stream capture: a call under capture records its uploads (seq_ids,
- *     n_tokens and the lists made of them; sequence state and page tables
- *     that changed since the last launch) as copies from staging memory that
- *     later calls reuse. Capture only calls that upload nothing - nda_decode,
- *     nda_step, nda_attention and nda_attention_block of sequences 0..n-1,
- *     after a first call outside the capture at the same positions - and
- *     replay only while the context's buffers have not grown. A call outside
- *     the graph is right whatever was captured and replayed before it.
+ *     n_tokens and the lists made of them, the shared-prefix pass's among
+ *     them; sequence state and page tables that changed since the last
+ *     launch) as copies from staging memory that later calls reuse. Capture
+ *     only calls that upload nothing - nda_decode, nda_step, nda_attention
+ *     and nda_attention_block of sequences 0..n-1 not all on one shared
+ *     prefix - after the same call outside the capture on the same stream at
+ *     the same positions, and replay only while the context's buffers have
+ *     not grown. A call outside the graph is right whatever was captured and
+ *     replayed before it.
  */
 #ifndef NDA_H
 #define NDA_H

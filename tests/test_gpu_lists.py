@@ -164,3 +164,57 @@ def test_lists_of_every_kind(streams):
     if streams > 1:
         for s in st:
             N._check(N.lib().nda_stream_destroy(s))
+
+
+@pytest.mark.parametrize("kv,nh,nkv,qk,n", [("int8", 12, 2, 48, 40), ("int8", 12, 2, 48, 700), ("f16", 8, 8, 64, 20)])
+def test_captured_steps(kv, nh, nkv, qk, n):
+    """nda_step and nda_decode of sequences 0..n-1 in a graph (700 sequences:
+    the launch that goes longest row first outside of one): every replay,
+    between eager calls with listed ids and other row counts, equals the
+    eager result."""
+    N = nda()
+    hip = N.C.CDLL("libamdhip64.so")
+
+    def ok(rc):
+        assert rc == 0, rc
+
+    st, graph, ex = N.vp(), N.vp(), N.vp()
+    N._check(N.lib().nda_stream_create(N.C.byref(st)))
+    ctx = N.Context(1, nh, nkv, qk, VD, 320, kv_dtype=N.KV_F16 if kv == "f16" else N.KV_INT8, max_seqs=n)
+    for b in range(n):
+        ctx.seq_set_pos(b, (37 * b) % 300)
+    ctx.kv_fill_normal(n, seed=3, stream=st)
+    rng = np.random.default_rng(n)
+    q, k, v = ([N.DevBuf.from_array(rng.standard_normal((n, h, d)).astype(np.float32)) for _ in range(2)]
+               for h, d in ((nh, qk), (nkv, qk), (nkv, VD)))
+    outs = [N.DevBuf(n * nh * VD * 4) for _ in range(3)]
+
+    def calls(o):
+        ctx.step(0, n, q[0], k[0], v[0], outs[o], stream=st)
+        ctx.decode(0, n, q[1], outs[o + 1], stream=st)
+
+    calls(0)
+    ctx.sync(st)
+    want = [outs[o].to_array(np.uint32, (n, nh, VD)) for o in (0, 1)]
+    ok(hip.hipStreamBeginCapture(st, 2))
+    calls(0)
+    ok(hip.hipStreamEndCapture(st, N.C.byref(graph)))
+    ok(hip.hipGraphInstantiate(N.C.byref(ex), graph, None, None, N.C.c_size_t(0)))
+    for rep in range(4):
+        ids = [int(x) for x in rng.permutation(n)[:n // (rep + 1)]]
+        ctx.decode(0, len(ids), q[rep % 2], outs[2], seq_ids=ids, stream=st)
+        ctx.sync(st)
+        listed = outs[2].to_array(np.uint32, (len(ids), nh, VD))
+        for o in (0, 1):
+            outs[o].upload(np.zeros((n, nh, VD), np.float32))
+        ok(hip.hipGraphLaunch(ex, st))
+        ctx.sync(st)
+        for o in (0, 1):
+            assert np.array_equal(outs[o].to_array(np.uint32, (n, nh, VD)), want[o]), (rep, o)
+        ctx.decode(0, len(ids), q[rep % 2], outs[2], seq_ids=ids, stream=st)
+        ctx.sync(st)
+        assert np.array_equal(outs[2].to_array(np.uint32, (len(ids), nh, VD)), listed), rep
+    ok(hip.hipGraphExecDestroy(ex))
+    ok(hip.hipGraphDestroy(graph))
+    ctx.close()
+    N._check(N.lib().nda_stream_destroy(st))
