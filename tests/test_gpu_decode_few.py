@@ -128,6 +128,18 @@ def test_valu_waves(nh, nkv, qk, f16, n, fused):
     check(nh, nkv, qk, f16, [n, n, n], n, fused=fused)
 
 
+# 3 rows; one item per CU and one more, two and one more: where the least
+# length for eight waves changes (rep 8: 128, 256 and 512 positions)
+@pytest.mark.parametrize("nh,nkv,qk,f16,rows,n", [
+    (8, 2, 64, True, 3, 128), (14, 2, 64, True, 3, 128), (16, 2, 64, True, 3, 300), (21, 3, 48, False, 3, 200),
+    (16, 2, 64, True, 128, 128), (16, 2, 64, True, 129, 255), (16, 2, 64, True, 129, 256), (16, 2, 64, True, 257, 511),
+    (16, 2, 64, True, 257, 512), (10, 2, 36, False, 200, 170),
+])
+@pytest.mark.parametrize("fused", [True, False])
+def test_valu_waves_by_heads(nh, nkv, qk, f16, rows, n, fused):
+    check(nh, nkv, qk, f16, [n - 1] * rows, n, fused=fused)
+
+
 def test_valu_chunks():
     """Long rows in chunks, int8 and fp16, where the MFMA decode does not go."""
     for f16 in (True, False):
